@@ -94,8 +94,8 @@ def batched_section(steps, seq_cases):
     batch (FP16-shift storage, FP32 collision, autotuned tiles) against the
     same cases solved one at a time as plain lattices, in the same storage
     format (the gain of batching) and in FP64 (a sample of `seq_cases`,
-    scaled by nodes).  The lone lattices take their fastest step, the
-    temporally blocked one where their timing picks it."""
+    scaled by nodes).  Batch and lone lattices take temporally blocked steps
+    by their size."""
     import tclb_amd
     from tclb_amd import cases
     model = "d2q9_drag"
@@ -169,13 +169,13 @@ def serving_section(rate, window, sample, nsat):
 def cylinder_section(steps):
     """The 1024x128 d2q9 cylinder in FP64 with the drag/lift Globals on the
     last step of each 1000-step segment; plain steps as the lattice chooses
-    by timing (`temporal_blocking`: steps per launch, 0 for single steps)."""
+    by its size (`temporal_blocking`: steps per launch, 0 for single steps)."""
     import tclb_amd
     from tclb_amd import cases
     c = cases.d2q9_cylinder(steps=steps)
     lat = c.build("f64")
     lat.prepare()
-    lat.iterate(400)   # its first 270 steps time the temporal blocking
+    lat.iterate(400)
     t0 = time.perf_counter()
     for _ in range(steps // 1000):
         lat.iterate(1000)

@@ -232,21 +232,18 @@ int tclbx_get_sorted_dispatch(tclbx_lattice* h, int* on, long long* list_nodes);
 int tclbx_set_stochastic_rounding(tclbx_lattice* h, int on, unsigned seed);
 /* Temporal blocking of the plain steps of the 2D models d2q9_SRT,
  * d2q9_SRT_drag, d2q9 and d2q9_drag (TCLBX_ERR for the others): `steps`
- * (2-15) time steps per launch, each block stepping a 32 x 32 tile with
- * `steps` nodes of halo in LDS and writing its interior; 0 or 1 turns it
- * off; -1, the default of these models, lets a lattice under 2^23 nodes
- * time single steps against 3 and 5 per launch on the first 270 plain steps
- * of the first tclbx_iterate that runs that many (real steps of the run)
- * and keep the fastest.  Results
- * are those of single steps, bit for bit, stochastic rounding included.
- * Steps with Globals take the single step.  It pays where one step does
- * not fill the GPU or the snapshots sit in the Infinity Cache, and loses
- * where steps stream from HBM.  The environment's TCLBX_TEMPORAL_BLOCKING=k
- * (k >= 0) fixes it for new lattices of these models.  No counterpart in
- * the reference, which launches one kernel per iteration
- * (src/Lattice.cu.Rt:1246-1297). */
+ * (2-15) time steps per launch, on tiles held in LDS or, up to 5 steps on
+ * larger lattices, by waves that march through the lattice with the steps
+ * in between in registers; 0 or 1 turns it off; -1, the default of these
+ * models, takes the steps per launch that the lattice's size and storage
+ * format call for when it first iterates.  Results are those of single
+ * steps, bit for bit, stochastic rounding included.  Steps with Globals take
+ * the single step.  Batches of these models step the same way.  The
+ * environment's TCLBX_TEMPORAL_BLOCKING=k (k >= 0) fixes it for new
+ * lattices and batches.  No counterpart in the reference, which launches
+ * one kernel per iteration (src/Lattice.cu.Rt:1246-1297). */
 int tclbx_set_temporal_blocking(tclbx_lattice* h, int steps);
-/* the steps per launch in use (0: single steps, also before a timed choice) */
+/* the steps per launch in use (0: single steps, also before the first tclbx_iterate chose) */
 int tclbx_get_temporal_blocking(tclbx_lattice* h, int* steps);
 
 /* ---------------------------------------------------------------- batch --

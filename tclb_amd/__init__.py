@@ -538,10 +538,10 @@ class Lattice:
     @property
     def temporal_blocking(self):
         """Plain steps per launch of the temporally blocked 2D step in use (0:
-        single steps).  Set k >= 2 to fix it, 0 to turn it off, -1 to let
-        the lattice time 1, 3 and 5 steps per launch on the first 270 plain
-        steps of its first Iterate that runs that many and keep the fastest
-        (the default of d2q9_SRT, d2q9_SRT_drag, d2q9 and d2q9_drag)."""
+        single steps).  Set k >= 2 to fix it, 0 to turn it off, -1 to take
+        the number the lattice's size and storage format call for (the
+        default of d2q9_SRT, d2q9_SRT_drag, d2q9 and d2q9_drag, chosen when
+        the lattice first iterates)."""
         k = ctypes.c_int()
         _check(lib().tclbx_get_temporal_blocking(self._h, ctypes.byref(k)))
         return k.value

@@ -2,6 +2,7 @@
 #include "batch.h"
 
 #include <algorithm>
+#include <cstdlib>
 #include <cstring>
 #include <limits>
 #include <stdexcept>
@@ -74,6 +75,10 @@ const ModelDef* batchable(const ModelDef* m, int storage) {
 Batch::Batch(const ModelDef* m, int storage_, size_t capacity_bytes)
     : model(batchable(m, storage_)), storage(storage_), arena_(capacity_bytes) {
     graph_steps_ = default_graph_steps();
+    // plain steps of a 2D model per launch: by the batch's size, or as the
+    // environment fixes it for lattices and batches (0 and 1: single steps)
+    if (const char* e = std::getenv("TCLBX_TEMPORAL_BLOCKING"))
+        if (std::atoi(e) >= 0) tb_k_ = std::max(1, std::min(TB_MAX_K, std::atoi(e)));
     hip_check(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking), "hipStreamCreate");
     hip_check(hipEventCreate(&ev0_), "hipEventCreate");
     hip_check(hipEventCreate(&ev1_), "hipEventCreate");
@@ -90,8 +95,8 @@ Batch::~Batch() {
     drop_graph();
     for (auto& kv : active_)
         if (kv.second.d_zone) (void)hipFree(kv.second.d_zone);
-    for (void* p : {(void*)d_cases_, (void*)d_tiles_, (void*)d_gtiles_, (void*)d_first_, (void*)d_count_,
-                    (void*)d_gpart_, (void*)d_glob_})
+    for (void* p : {(void*)d_cases_, (void*)d_tiles_, (void*)d_gtiles_, (void*)d_bitems_, (void*)d_first_,
+                    (void*)d_count_, (void*)d_gpart_, (void*)d_glob_})
         if (p) (void)hipFree(p);
     if (ev0_) (void)hipEventDestroy(ev0_);
     if (ev1_) (void)hipEventDestroy(ev1_);
@@ -278,15 +283,22 @@ void Batch::InitCase(int id) {
 // lists, and per case the slice of Globals tiles it reduces
 void Batch::rebuild() {
     drop_graph();
-    for (void* p : {(void*)d_cases_, (void*)d_tiles_, (void*)d_gtiles_, (void*)d_first_, (void*)d_count_,
-                    (void*)d_gpart_, (void*)d_glob_})
+    for (void* p : {(void*)d_cases_, (void*)d_tiles_, (void*)d_gtiles_, (void*)d_bitems_, (void*)d_first_,
+                    (void*)d_count_, (void*)d_gpart_, (void*)d_glob_})
         if (p) (void)hipFree(p);
-    d_cases_ = nullptr; d_tiles_ = d_gtiles_ = nullptr; d_first_ = d_count_ = nullptr;
+    d_cases_ = nullptr; d_tiles_ = d_gtiles_ = d_bitems_ = nullptr; d_first_ = d_count_ = nullptr;
     d_gpart_ = d_glob_ = nullptr;
     order_.clear();
     std::vector<BatchCase> descs;
-    std::vector<int2> tiles, gtiles;
+    std::vector<int2> tiles, gtiles, bitems;
     std::vector<int> first, count;
+    blocked_ = BlockedBatch();
+    std::vector<Blocking> split(active_.size());
+    if (tb_k_ != 1 && !active_.empty() && blocked2d_model(model->id)) {
+        std::vector<int2> sizes;
+        for (auto& kv : active_) sizes.push_back(make_int2(kv.second.nx, kv.second.ny));
+        blocked_ = blocking2d_batch(sizes.data(), (int)sizes.size(), storage, tb_k_, split.data());
+    }
     for (auto& kv : active_) {
         const Case& c = kv.second;
         const int slot = (int)order_.size();
@@ -297,6 +309,12 @@ void Batch::rebuild() {
         bc.parity = c.parity;
         bc.sr_iter = (unsigned)c.iter;
         bc.sr_seed = sr_seed_;
+        if (blocked_.k > 1) {
+            const Blocking& b = split[slot];
+            bc.args.tb_k = b.k; bc.args.tb_rows = b.rows; bc.args.tb_tx = b.tx; bc.args.tb_ty = b.ty;
+            const int nb = blocked2d_items(bc.args);
+            for (int t = 0; t < nb; t++) bitems.push_back(make_int2(slot, t));
+        }
         descs.push_back(bc);
         const int nt = step_blocks(bc.args, false, tune_.block);
         for (int t = 0; t < nt; t++) tiles.push_back(make_int2(slot, t));
@@ -307,12 +325,18 @@ void Batch::rebuild() {
     }
     ntiles_ = (int)tiles.size();
     ngtiles_ = (int)gtiles.size();
+    nbitems_ = (int)bitems.size();
     ncases_dev_ = (int)descs.size();
     const int G = kernel_nglobals(model->id);
     if (ncases_dev_ > 0) {
         hip_check(hipMalloc((void**)&d_cases_, descs.size() * sizeof(BatchCase)), "hipMalloc(cases)");
         hip_check(hipMalloc((void**)&d_tiles_, tiles.size() * sizeof(int2)), "hipMalloc(tiles)");
         hip_check(hipMalloc((void**)&d_gtiles_, gtiles.size() * sizeof(int2)), "hipMalloc(tiles)");
+        if (nbitems_ > 0) {
+            hip_check(hipMalloc((void**)&d_bitems_, bitems.size() * sizeof(int2)), "hipMalloc(blocked items)");
+            hip_check(hipMemcpy(d_bitems_, bitems.data(), bitems.size() * sizeof(int2), hipMemcpyHostToDevice),
+                      "upload blocked items");
+        }
         hip_check(hipMalloc((void**)&d_first_, first.size() * sizeof(int)), "hipMalloc(first)");
         hip_check(hipMalloc((void**)&d_count_, count.size() * sizeof(int)), "hipMalloc(count)");
         hip_check(hipMalloc((void**)&d_gpart_, (size_t)ngtiles_ * G * 2 * sizeof(double)), "hipMalloc(partials)");
@@ -353,6 +377,20 @@ void Batch::launch(int phase, bool glob, int k) {
     }
 }
 
+// `steps` plain steps in one launch; the first is step k of the Iterate
+hipError_t Batch::launch_blocked(int phase, int steps, int k) {
+    const int st = !sr_ ? storage : (storage == ST_F16S ? ST_F16S_SR : ST_BF16S_SR);
+    return launch_blocked_batch(model->id, st, d_cases_, d_bitems_, nbitems_, (phase & 1) | (k << 2), steps, blocked_,
+                                stream_);
+}
+
+// steps of one replay of the captured loop: graph_steps_, or with blocked
+// steps an even number (at least two) of launches
+int Batch::graph_len() const {
+    if (blocked_.k == 1) return graph_steps_;
+    return std::max(2, (graph_steps_ / blocked_.k) & ~1) * blocked_.k;
+}
+
 void Batch::drop_graph() {
     if (graph_exec_) (void)hipGraphExecDestroy(graph_exec_);
     if (graph_) (void)hipGraphDestroy(graph_);
@@ -361,16 +399,18 @@ void Batch::drop_graph() {
     graph_version_ = ~0u;
 }
 
-// graph_steps_ plain steps from phase 0, captured once per set of cases
+// graph_len() plain steps from phase 0, captured once per set of cases
 void Batch::capture_graph() {
     if (graph_exec_ != nullptr && graph_version_ == version_) return;
     drop_graph();
     hip_check(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal), "begin capture");
-    for (int k = 0; k < graph_steps_; k++) {
+    for (int k = 0; k < graph_len() / blocked_.k; k++) {
         const int nt = ntiles_;
         const int grid = tune_.grid > 0 ? std::min(tune_.grid, nt) : nt;
-        hipError_t e = launch_batch_step(model->id, storage, false, d_cases_, d_tiles_, nt,
-                                         (k & 1) | (tune_.order ? 2 : 0), d_gpart_, grid, tune_.block, stream_);
+        hipError_t e = blocked_.k > 1 ? launch_blocked(k & 1, blocked_.k, 0)
+                                      : launch_batch_step(model->id, storage, false, d_cases_, d_tiles_, nt,
+                                                          (k & 1) | (tune_.order ? 2 : 0), d_gpart_, grid,
+                                                          tune_.block, stream_);
         if (e != hipSuccess) {
             hipGraph_t g = nullptr;
             (void)hipStreamEndCapture(stream_, &g);
@@ -420,18 +460,29 @@ void Batch::Iterate(int niter, int iter_type) {
     int i = 0;
     const int plain_end = niter - (last_glob ? 1 : 0);
     const bool captured = graph_exec_ != nullptr && graph_version_ == version_;
-    const int lead = phase_ != 0 ? 1 : 0;
+    const int k = every_glob ? 1 : blocked_.k, glen = graph_len();
+    const int lead = phase_ != 0 ? k : 0;
     if (sr_) upload_sr_iterations();
-    if (!every_glob && !sr_ && graph_steps_ >= 2 && plain_end - lead >= (captured ? 1 : 2) * graph_steps_) {
+    if (!every_glob && !sr_ && graph_steps_ >= 2 && plain_end - lead >= (captured ? 1 : 2) * glen) {
         if (phase_ != 0) {
-            launch(phase_, false);
+            if (k > 1) hip_check(launch_blocked(phase_, k, i), "blocked batch step");
+            else launch(phase_, false);
             phase_ ^= 1;
-            i++;
+            i += k;
         }
         capture_graph();
-        const int reps = (plain_end - i) / graph_steps_;
+        const int reps = (plain_end - i) / glen;
         for (int r = 0; r < reps; r++) hip_check(hipGraphLaunch(graph_exec_, stream_), "graph launch");
-        i += reps * graph_steps_;
+        i += reps * glen;
+    }
+    // the remaining plain steps: tiles take any number up to k, spread
+    // evenly, marching waves k at a time (fewer than that launch below)
+    while (k > 1 && plain_end - i >= (blocked_.rows > 0 ? k : 2)) {
+        const int left = plain_end - i, launches = (left + k - 1) / k;
+        const int kk = blocked_.rows > 0 ? k : (left + launches - 1) / launches;
+        hip_check(launch_blocked(phase_, kk, i), "blocked batch step");
+        phase_ ^= 1;
+        i += kk;
     }
     for (; i < niter; i++) {
         const bool glob = every_glob || (last_glob && i == niter - 1);

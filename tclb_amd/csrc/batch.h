@@ -132,6 +132,8 @@ private:
     void upload_sr_iterations();
     void drop_graph();
     void capture_graph();
+    hipError_t launch_blocked(int phase, int steps, int k);
+    int graph_len() const;
     Case& get(int id);
     const Case& get(int id) const;
 
@@ -149,11 +151,16 @@ private:
     BatchCase* d_cases_ = nullptr;
     int2* d_tiles_ = nullptr;
     int2* d_gtiles_ = nullptr;
+    int2* d_bitems_ = nullptr;   // blocked steps: {case, tile or strip of the case}
     int* d_first_ = nullptr;
     int* d_count_ = nullptr;
     double* d_gpart_ = nullptr;
     double* d_glob_ = nullptr;
-    int ntiles_ = 0, ngtiles_ = 0, ncases_dev_ = 0;
+    int ntiles_ = 0, ngtiles_ = 0, nbitems_ = 0, ncases_dev_ = 0;
+    // plain steps per launch of a 2D batch: tb_k_ = 0 by size, else fixed (1:
+    // single steps); blocked_ is what the current set of cases got
+    int tb_k_ = 0;
+    BlockedBatch blocked_;
     std::vector<int> order_;  // case id of device slot i
     hipStream_t stream_ = nullptr;
     hipEvent_t ev0_ = nullptr, ev1_ = nullptr;

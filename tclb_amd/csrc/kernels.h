@@ -16,9 +16,10 @@ namespace tclbx {
 // d3q27_cumulant and its builds: [nu, nubuffer, GalileanCorrection, ForceX,
 // ForceY, ForceZ, Omega, Smag].
 constexpr int MAX_PAR = 16;
-// side of the tiles of the temporally blocked step (nodes, one per thread);
-// it takes at most TB_TILE / 2 - 1 steps per launch
-constexpr int TB_TILE = 32;
+// the temporally blocked 2D step takes at most TB_MAX_K steps per launch (a
+// tile of 1,024 nodes then still has a middle to write)
+constexpr int TB_MAX_K = 15;
+constexpr int MARCH2D_MAX_K = 5, TILE2D_MAX_TX = 64;
 constexpr int MAX_GLOBALS = 32;
 
 struct StepArgs {
@@ -46,13 +47,16 @@ struct StepArgs {
     // below the zone) is bulk_val, the plain collision node, so that every
     // wavefront takes the same branch; mode 2 the list[0..list_n) of the
     // other nodes, sorted by class, one thread each.  Mode 3: tb_k plain
-    // steps in one launch of the temporally blocked step (2D models), tiles
-    // of TB_TILE x TB_TILE nodes, tb_bx of them along x (set by the launch)
+    // steps in one launch of the temporally blocked step (2D models), as
+    // the tb_* fields below say (a Blocking of blocking2d)
     int mode;
     unsigned class_mask, bulk_val;
     const unsigned* list;
     unsigned list_n;
-    int tb_k, tb_bx;
+    int tb_k;
+    int tb_rows;        // marching waves: rows each wave writes; 0: LDS tiles
+    int tb_tx, tb_ty;   // LDS tiles: nodes along x and y
+    int tb_nt;          // LDS tiles: stores past the L2
     // stochastic rounding of the stores of a 16-bit format (0: nearest even);
     // sr_key = sr_key(iteration the step computes, the lattice's seed)
     int sr;
@@ -79,6 +83,30 @@ struct BatchCase {
     unsigned sr_iter, sr_seed;
     int pad_;
 };
+
+// The split of a temporally blocked 2D launch: marching waves (rows > 0) or
+// LDS tiles (tx x ty), up to k steps of either.
+struct Blocking {
+    int k = 1, rows = 0, tx = 0, ty = 0, nt = 0;
+};
+// the models the blocked steps cover
+bool blocked2d_model(int model);
+// The split for a lattice of nx x ny nodes: of k steps per launch, or with k =
+// 0 of the best number of steps (kernels.hip says why the lines lie there).
+Blocking blocking2d(int nx, int ny, int storage, int k);
+// The same for the lattices of a batch (nx, ny), which share the number of
+// steps, the kind and the block; each lattice's split goes to `cases`.
+struct BlockedBatch {
+    int k = 1, rows = 0, threads = 0;  // rows > 0: marching waves
+};
+BlockedBatch blocking2d_batch(const int2* sizes, int n, int storage, int k, Blocking* cases);
+// tiles, or strips of waves, of one lattice in a blocked launch
+int blocked2d_items(const StepArgs& a);
+// `steps` (2 to b.k; b.k exactly for marching waves) plain steps of every
+// lattice of a batch, one item {case, tile or strip of the case} per block or
+// wave; `phase` as launch_batch_step, with the first step's index
+hipError_t launch_blocked_batch(int model, int storage, const BatchCase* cases, const int2* items, int nitems,
+                                int phase, int steps, const BlockedBatch& b, hipStream_t s);
 
 // Blocks (tiles) of one step launch of the lattice `a` with `block`
 // threads per block (a Globals step walks a.rpb rows per block).

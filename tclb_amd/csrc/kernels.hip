@@ -4,6 +4,10 @@
 // compile unit of its family (kernels_<family>.hip).
 #include "kernels_impl.h"
 
+#include <algorithm>
+#include <cmath>
+#include <vector>
+
 namespace tclbx {
 
 // the compile unit of a family that holds the kernels of this storage format
@@ -115,6 +119,125 @@ double weight(int model, int q) {
     return (model == MODEL_D3Q19 || model == MODEL_D3Q19_LID) ? Lat<MODEL_D3Q19>::w(q) : Lat<MODEL_D2Q9_SRT>::w(q);
 }
 }  // namespace
+
+// Lines measured on d2q9_SRT in f64 and f32s and on d2q9_drag in f16s (us per
+// step, tiles against marching waves at each one's best split):
+//   f64   1501x333 8.8 / 10.6, 2048x512 17.8 / 15.6, 2048x1024 31.5 / 27.7,
+//         4096x2048 122 / 95
+//   f32s  2048x1024 13.3 / 14.3, 4096x2048 52.4 / 43.6
+//   f16s  2048x1024 14.4 / 15.3, 4096x2048 54.6 / 44.6
+// The waves need 3,000 or more of them to cover each other's latencies, each
+// with enough rows to pay for the 2(k-1) it steps beside them; the FP64 tile
+// holds one or two blocks per CU, the float tiles twice as many.
+static bool blocking2d_marches(long long nodes, int storage) {
+    return nodes >= (storage == ST_F64 ? 1ll << 20 : 1ll << 22);
+}
+
+static int strips2d(int nx, int k) { return (nx + 64 - 2 * (k - 1) - 1) / (64 - 2 * (k - 1)); }
+
+// Marching waves for n lattices of `nodes` nodes in all.
+// f64 4096x2048: k 3 104, 4 98, 5 95 us per step; 2048x1024: k 3 30.6, 4 27.7,
+// 5 30.5.  f32s 4096x2048: 60, 50, 44.  f16s: 44.6, 46.7, 50.5 (its
+// conversions make a step dearer than the bytes it saves).  Rows for about
+// 3,000 waves, between what pays for the extra rows and what evens out the
+// last round (f64 8-12 to 24, float 8 to 12 measured).
+static BlockedBatch march_split(const int2* sizes, int n, long long nodes, int storage, int k, Blocking* cases) {
+    const bool f64 = storage == ST_F64, half = storage == ST_F16S || storage == ST_BF16S;
+    BlockedBatch b;
+    b.k = k ? k : f64 ? (nodes >= 1ll << 22 ? 5 : 4) : half ? 3 : 5;
+    long long rows = 0;
+    for (int i = 0; i < n; i++) rows += (long long)strips2d(sizes[i].x, b.k) * sizes[i].y;
+    b.rows = (int)std::min<long long>(f64 ? 24 : 12, std::max<long long>(f64 ? 6 : 8, (rows + 3071) / 3072));
+    b.threads = 256;
+    for (int i = 0; i < n; i++) {
+        cases[i] = Blocking();
+        cases[i].k = b.k;
+        cases[i].rows = std::min(b.rows, sizes[i].y);
+    }
+    return b;
+}
+
+// The tiles of the least estimated time per step.  A launch takes rounds x (A
+// + k x stage), stage = s0 + s1 x waves per SIMD, fitted to single rounds of
+// 128x32 and 1024x128 (f64: 16x16 tiles, one wave per SIMD, 0.84 us a stage,
+// 32x16 1.33, 32x32 2.25; f32s 0.55, 1.06, 1.37; f16s 0.83, -, 2.1) and to
+// the rounds of 1501x333 (f64 32x16, two rounds of 12.5 us at k = 3).
+static BlockedBatch tile_split(const int2* sizes, int n, int storage, const std::vector<int>& ks, Blocking* cases) {
+    const double A = 2.8, s0 = 0.4, s1 = storage == ST_F64 ? 0.47 : storage == ST_F32 || storage == ST_F32S ? 0.22 : 0.26;
+    const int capacity = storage == ST_F64 ? 6 : 8;   // waves per SIMD
+    std::vector<Blocking> trial(n);
+    BlockedBatch best;
+    double best_t = 1e300;
+    for (int k : ks)
+        for (int threads : {256, 512, 1024}) {
+            long long tiles = 0;
+            for (int i = 0; i < n && tiles >= 0; i++) {
+                long long fewest = 0;
+                // the widest of the shapes with the fewest tiles: its rows
+                // are longer runs of memory (1024x128 in FP64: 256 tiles
+                // of 40x25 3.1 us per step, of 24x42 3.6)
+                for (int tx : {TILE2D_MAX_TX, 56, 48, 44, 40, 36, 32, 28, 24, 20, 16}) {
+                    const int ty = threads / tx, wx = tx - 2 * (k - 1), wy = ty - 2 * (k - 1);
+                    if (wx < 1 || wy < 1) continue;
+                    const long long t = (long long)((sizes[i].x + wx - 1) / wx) * ((sizes[i].y + wy - 1) / wy);
+                    if (fewest == 0 || t < fewest) {
+                        fewest = t;
+                        trial[i].k = k; trial[i].rows = 0; trial[i].tx = tx; trial[i].ty = ty;
+                    }
+                }
+                tiles = fewest ? tiles + fewest : -1;
+            }
+            if (tiles < 0) continue;   // no tile of this many nodes has a middle
+            const int waves = threads / 256, fit = std::max(1, capacity / waves);   // blocks a CU holds
+            const long long per_cu = (tiles + 255) / 256;
+            double rounds = (double)tiles / (256.0 * fit);
+            rounds = rounds < 4 ? std::ceil(rounds) : rounds + 0.5;
+            const double t = rounds * (A + k * (s0 + s1 * waves * std::min<long long>(fit, per_cu))) / k;
+            if (t < best_t) {
+                best_t = t;
+                best.k = k; best.rows = 0; best.threads = threads;
+                for (int i = 0; i < n; i++) {
+                    cases[i] = trial[i];
+                    cases[i].nt = per_cu <= fit;
+                }
+            }
+        }
+    return best;
+}
+
+Blocking blocking2d(int nx, int ny, int storage, int k) {
+    const int2 size = make_int2(nx, ny);
+    Blocking b;
+    if (k <= MARCH2D_MAX_K && blocking2d_marches((long long)nx * ny, storage))
+        march_split(&size, 1, (long long)nx * ny, storage, k, &b);
+    else
+        tile_split(&size, 1, storage, k ? std::vector<int>{k} : std::vector<int>{3, 5}, &b);
+    return b;
+}
+
+BlockedBatch blocking2d_batch(const int2* sizes, int n, int storage, int k, Blocking* cases) {
+    long long nodes = 0;
+    for (int i = 0; i < n; i++) nodes += (long long)sizes[i].x * sizes[i].y;
+    if (k <= MARCH2D_MAX_K && blocking2d_marches(nodes, storage)) return march_split(sizes, n, nodes, storage, k, cases);
+    return tile_split(sizes, n, storage, k ? std::vector<int>{k} : std::vector<int>{3, 4, 5}, cases);
+}
+
+int blocked2d_items(const StepArgs& a) {
+    if (a.tb_rows > 0) return strips2d(a.nx, a.tb_k) * ((a.ny + a.tb_rows - 1) / a.tb_rows);
+    const int wx = a.tb_tx - 2 * (a.tb_k - 1), wy = a.tb_ty - 2 * (a.tb_k - 1);
+    if (wx < 1 || wy < 1) return 0;
+    return ((a.nx + wx - 1) / wx) * ((a.ny + wy - 1) / wy);
+}
+
+bool blocked2d_model(int model) {
+    return model == MODEL_D2Q9_SRT || model == MODEL_D2Q9_SRT_DRAG || model == MODEL_D2Q9 || model == MODEL_D2Q9_DRAG;
+}
+
+hipError_t launch_blocked_batch(int model, int storage, const BatchCase* cases, const int2* items, int nitems,
+                                int phase, int steps, const BlockedBatch& b, hipStream_t s) {
+    const hipError_t e = TCLBX_PICK(blocked_batch_2d, storage)(model, storage, cases, items, nitems, phase, steps, b, s);
+    return e == hipErrorNotFound ? hipErrorInvalidValue : e;
+}
 
 int step_blocks(const StepArgs& a, bool globals, int block) {
     const int rpb = globals ? a.rpb : a.rpt;

@@ -1,7 +1,7 @@
 // kernels_2d.hip -- instantiates and dispatches the node kernels of one
 // family of models (see kernels_impl.h); compiled apart so the families
 // build in parallel.
-#include "kernels_impl.h"
+#include "kernels_march.h"
 
 namespace tclbx {
 
@@ -63,6 +63,17 @@ hipError_t TCLBX_FAM(quantity_2d)(int model, int storage, int q, const StepArgs&
     case MODEL_D2Q9_BC: return quantity_m<MODEL_D2Q9_BC>(storage, q, a, x0, y0, z0, rx, ry, rz, scale, out, s);
     case MODEL_D2Q9_BC_AUTOSYM: return quantity_m<MODEL_D2Q9_BC_AUTOSYM>(storage, q, a, x0, y0, z0, rx, ry, rz, scale, out, s);
     case MODEL_D2Q9_BC_AUTOSYM2: return quantity_m<MODEL_D2Q9_BC_AUTOSYM2>(storage, q, a, x0, y0, z0, rx, ry, rz, scale, out, s);
+    }
+    return hipErrorNotFound;
+}
+
+hipError_t TCLBX_FAM(blocked_batch_2d)(int model, int storage, const BatchCase* cases, const int2* items, int nitems,
+                                       int phase, int steps, const BlockedBatch& b, hipStream_t s) {
+    switch (model) {
+    case MODEL_D2Q9_SRT: return blocked_batch2d_m<MODEL_D2Q9_SRT>(storage, cases, items, nitems, phase, steps, b, s);
+    case MODEL_D2Q9_SRT_DRAG: return blocked_batch2d_m<MODEL_D2Q9_SRT_DRAG>(storage, cases, items, nitems, phase, steps, b, s);
+    case MODEL_D2Q9: return blocked_batch2d_m<MODEL_D2Q9>(storage, cases, items, nitems, phase, steps, b, s);
+    case MODEL_D2Q9_DRAG: return blocked_batch2d_m<MODEL_D2Q9_DRAG>(storage, cases, items, nitems, phase, steps, b, s);
     }
     return hipErrorNotFound;
 }

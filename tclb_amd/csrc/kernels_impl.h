@@ -258,7 +258,8 @@ __device__ __forceinline__ void d2q9_feq(R* f_eq, R d, R ux, R uy) {
 // balance and the rest population from the mass balance.  Evaluated
 // directly, the rounded weights 1/9, 1/36 and an approximate 1/rho create
 // mass and momentum each step.
-__device__ __forceinline__ void d2q9_bgk_dev(float* d, float omega, const double* zr) {
+template <class Z>
+__device__ __forceinline__ void d2q9_bgk_dev(float* d, float omega, const Z& zr) {
     const float s = ((d[0] + d[1]) + (d[2] + d[3])) + ((d[4] + d[5]) + (d[6] + d[7])) + d[8];
     const float rho = 1.f + s;
     const float d57 = d[5] - d[7], d68 = d[6] - d[8];
@@ -283,8 +284,8 @@ __device__ __forceinline__ void d2q9_bgk_dev(float* d, float omega, const double
     d[5] += D5; d[6] += D6; d[7] += D7; d[8] += D8;
 }
 
-template <class R, bool DRAG, bool GLOB, bool COLLIDE = true>
-__device__ __forceinline__ void d2q9_node(R* f, unsigned nt, R omega, R Density, const double* zr,
+template <class R, bool DRAG, bool GLOB, bool COLLIDE = true, class Z>
+__device__ __forceinline__ void d2q9_node(R* f, unsigned nt, R omega, R Density, const Z& zr,
                                           double* g) {
     R uf;
     switch (nt & 0x7u) {
@@ -359,8 +360,8 @@ __device__ __forceinline__ void d2q9_node(R* f, unsigned nt, R omega, R Density,
 
 // d2q9_SRT node of a shifted storage format, on the deviations d = f - w:
 // boundary nodes add w back for their boundary condition, BGK runs on d.
-template <bool DRAG, bool GLOB>
-__device__ __forceinline__ void d2q9_node_dev(float* d, unsigned nt, float omega, float Density, const double* zr,
+template <bool DRAG, bool GLOB, class Z>
+__device__ __forceinline__ void d2q9_node_dev(float* d, unsigned nt, float omega, float Density, const Z& zr,
                                               double* g) {
     using L = Lat<MODEL_D2Q9_SRT>;
     if ((nt & 0x7u) != 0u) {
@@ -547,8 +548,8 @@ __device__ __forceinline__ void d2q9m_symmetry(R* f) {
 // non-equilibrium change.  DEV: f holds the deviations f - w, whose moments
 // are those of f except m0, which is rho - 1 (the rest populations w have
 // only the zeroth moment).  Zone columns and Globals as d2q9m_node.
-template <bool GLOB, bool DRAG, bool BCOPT, bool DEV>
-__device__ __forceinline__ void d2q9m_collide_f(float* f, unsigned nt, const double* par, const double* zr,
+template <bool GLOB, bool DRAG, bool BCOPT, bool DEV, class Z>
+__device__ __forceinline__ void d2q9m_collide_f(float* f, unsigned nt, const double* par, const Z& zr,
                                                 double* g, double* bc, size_t NN) {
     constexpr int OBJ = DRAG ? 5 : 3;
     float m[9];
@@ -606,8 +607,8 @@ __device__ __forceinline__ void d2q9m_collide_f(float* f, unsigned nt, const dou
 // DRAG adds the momentum exchange of Solid nodes, 2 sum_i f_i e_i of the
 // incoming populations (as d2q9_SRT_drag).  BCOPT: the bc builds, with the
 // node's BC[0] at bc[0] and BC[1] at bc[NN] (null: BC = 0, nothing kept).
-template <class R, bool GLOB, bool DRAG, bool BCOPT = false, bool COLLIDE = true>
-__device__ __forceinline__ void d2q9m_node(R* f, unsigned nt, const double* par, const double* zr, double* g,
+template <class R, bool GLOB, bool DRAG, bool BCOPT = false, bool COLLIDE = true, class Z>
+__device__ __forceinline__ void d2q9m_node(R* f, unsigned nt, const double* par, const Z& zr, double* g,
                                            double* bc = nullptr, size_t NN = 0) {
     constexpr int OBJ = DRAG ? 5 : 3;
     R Vx = (R)zr[0], Vy = (R)zr[1];
@@ -713,8 +714,8 @@ __device__ __forceinline__ void d2q9m_node(R* f, unsigned nt, const double* par,
 // d2q9 MRT node of a shifted storage format, on the deviations d = f - w:
 // boundary nodes add w back for their boundary condition, the collision
 // runs on d.
-template <bool GLOB, bool DRAG, bool BCOPT>
-__device__ __forceinline__ void d2q9m_node_dev(float* d, unsigned nt, const double* par, const double* zr,
+template <bool GLOB, bool DRAG, bool BCOPT, class Z>
+__device__ __forceinline__ void d2q9m_node_dev(float* d, unsigned nt, const double* par, const Z& zr,
                                                double* g, double* bc, size_t NN) {
     using L = Lat<MODEL_D2Q9_SRT>;
     if ((nt & 0xFu) != 0u) {
@@ -2191,120 +2192,6 @@ k_step_list(StepArgs a) {
     node_update<MODEL, ST, false, 0, true>(a, row, x, xm, xp, in, g);
 }
 
-// ------------------------------------------------- temporally blocked step ---
-// 2D models whose node update reads nothing but its own node's pulled
-// populations, flags and zone (no mirror nodes, no densities updated in
-// place): d2q9_SRT, d2q9_SRT_drag, d2q9 and d2q9_drag.
-template <int MODEL>
-constexpr bool tb_model = MODEL == MODEL_D2Q9_SRT || MODEL == MODEL_D2Q9_SRT_DRAG || MODEL == MODEL_D2Q9 ||
-                          MODEL == MODEL_D2Q9_DRAG;
-
-// The stored form of population i, rounded as the single step rounds its
-// store; with stochastic rounding direction 2j takes word j of the node's
-// stream and 2j + 1 word j << 16 (w advances after each odd direction).
-template <class S, class L, bool DEV>
-__device__ __forceinline__ typename S::T tb_stored(typename S::R v, int i, uint32_t& w) {
-    using R = typename S::R;
-    if constexpr (S::stochastic) {
-        const uint32_t r = (i & 1) ? w << 16 : w;
-        const typename S::T out = DEV ? S::unraw_sr(v, r) : S::put_sr(v, (R)L::w(i), r);
-        if (i & 1) w = xorshift32(w);
-        return out;
-    } else {
-        return DEV ? S::unraw(v) : S::put(v, (R)L::w(i));
-    }
-}
-
-// K = a.tb_k plain steps of a 2D lattice in one launch.  Block b takes the
-// TX x TY tile whose interior is the (TX - 2K) x (TY - 2K) nodes from
-// ((b % tb_bx)(TX - 2K), (b / tb_bx)(TY - 2K)), K nodes of halo on every
-// side (periodic wrap), loads its populations of the current snapshot into
-// LDS and steps the tile K times there.  After step s the nodes at least s
-// from the tile's edge hold exact values (their pulls reached only nodes
-// that held exact values), so the last step writes the interior to the
-// next snapshot.  Every pull of a step is read before any node writes its
-// own populations (a barrier between), so one LDS copy of the tile serves
-// all K steps.  Each value written to LDS is rounded to the storage format
-// exactly as the single step rounds its stores, and the node update is the
-// single step's own (stochastic rounding included: step s draws the words
-// of its own iteration): K launches of k_step and one of this give the
-// same bits.  The halo is computed again by the neighbouring blocks; the
-// launch saves K - 1 round trips through memory and K - 1 launch
-// latencies, which pays where a lattice is too small for one step to fill
-// the GPU.
-template <int MODEL, int ST, int TX, int TY>
-__global__ void __launch_bounds__(TX * TY) k_step_tb(StepArgs a) {
-    using L = Lat<MODEL>;
-    using S = Store<ST>;
-    using T = typename S::T;
-    using R = typename S::R;
-    constexpr int Q = 9;
-    constexpr bool DEV = S::shifted;
-    static_assert(tb_model<MODEL> && L::Q == 9, "2D models");
-    __shared__ T tile[Q][TY][TX];
-    const int K = a.tb_k;
-    const int nx = a.nx, ny = a.ny;
-    const int bx = blockIdx.x % a.tb_bx, by = blockIdx.x / a.tb_bx;
-    const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
-    // this thread's tile node: unwrapped coordinates (ux, uy), lattice node (x, y)
-    const int ux = bx * (TX - 2 * K) - K + tx, uy = by * (TY - 2 * K) - K + ty;
-    int x = ux % nx, y = uy % ny;
-    if (x < 0) x += nx;
-    if (y < 0) y += ny;
-    const unsigned n = (unsigned)x + (unsigned)nx * (unsigned)y;
-    const unsigned nt = *(gptr<const uint16_t>)(a.flags + n);
-    int zone = (int)(nt >> L::ZSHIFT);
-    if (zone >= a.nzones) zone = 0;
-    const double* zr = a.zone + (size_t)zone * a.zcols;
-    const size_t pbytes = (size_t)a.pitch * sizeof(T);
-    const char* fin = (const char*)a.fin;
-#pragma unroll
-    for (int i = 0; i < Q; i++) tile[i][ty][tx] = *(gptr<const T>)(fin + (size_t)i * pbytes + n * (unsigned)sizeof(T));
-    // the interior node this thread writes at the end (each lattice node is
-    // the interior node of exactly one tile)
-    const bool writes = tx >= K && tx < TX - K && ty >= K && ty < TY - K && ux < nx && uy < ny;
-    double g[1];
-    for (int s = 1; s <= K; s++) {
-        __syncthreads();
-        R f[Q];
-#pragma unroll
-        for (int i = 0; i < Q; i++) {
-            // the pull of the tile's edge nodes is clamped into the tile:
-            // their values are never used
-            const int sx = min(max(tx - L::ex(i), 0), TX - 1);
-            const int sy = min(max(ty - L::ey(i), 0), TY - 1);
-            const T v = tile[i][sy][sx];
-            f[i] = DEV ? S::raw(v) : S::get(v, (R)L::w(i));
-        }
-        __syncthreads();
-        if constexpr (is_d2q9m<MODEL> && DEV)
-            d2q9m_node_dev<false, MODEL == MODEL_D2Q9_DRAG, false>(f, nt, a.par, zr, g, nullptr, 0);
-        else if constexpr (is_d2q9m<MODEL>)
-            d2q9m_node<R, false, MODEL == MODEL_D2Q9_DRAG, false>(f, nt, a.par, zr, g, nullptr, 0);
-        else if constexpr (DEV)
-            d2q9_node_dev<MODEL == MODEL_D2Q9_SRT_DRAG, false>(f, nt, (R)a.par[0], (R)a.par[1], zr, g);
-        else
-            d2q9_node<R, MODEL == MODEL_D2Q9_SRT_DRAG, false>(f, nt, (R)a.par[0], (R)a.par[1], zr, g);
-        // stochastic rounding: the words of this node at the iteration
-        // step s computes, as the single step of that iteration draws them
-        uint32_t w = 0;
-        if constexpr (S::stochastic) w = sr_word0(n, sr_key(a.sr_step + (unsigned)(s - 1), a.sr_seed));
-        if (s < K) {
-#pragma unroll
-            for (int i = 0; i < Q; i++) tile[i][ty][tx] = tb_stored<S, L, DEV>(f[i], i, w);
-        } else if (writes) {
-            char* fout = (char*)a.fout;
-#pragma unroll
-            for (int i = 0; i < Q; i++)
-                __builtin_nontemporal_store(tb_stored<S, L, DEV>(f[i], i, w),
-                                            (gptr<T>)(fout + (size_t)i * pbytes + n * (unsigned)sizeof(T)));
-        }
-    }
-}
-
-// tile of the temporally blocked step: 32 x 32 nodes, one per thread
-constexpr int TB_TX = TB_TILE, TB_TY = TB_TILE;
-
 // waves per SIMD the plain step of MODEL in storage ST is held to (0: none)
 template <int MODEL, int ST>
 constexpr int step_waves() {
@@ -2609,22 +2496,25 @@ __global__ void __launch_bounds__(256) k_quantity(StepArgs a, int qid, int x0, i
 }
 
 // ------------------------------------------------------ launch templates ---
+// the temporally blocked step of a 2D model (kernels_march.h, compiled with
+// the 2D family only)
+template <int MODEL, int ST>
+hipError_t blocked2d_ms(const StepArgs& a, hipStream_t s);
+// 2D models whose node update reads nothing but its own node's pulled
+// populations, flags and zone (no mirror nodes, no densities updated in
+// place)
+template <int MODEL>
+constexpr bool tb_model = MODEL == MODEL_D2Q9_SRT || MODEL == MODEL_D2Q9_SRT_DRAG || MODEL == MODEL_D2Q9 ||
+                          MODEL == MODEL_D2Q9_DRAG;
+
 inline int nblocks_of(const StepArgs& a, int block) { return a.bpr * a.ny * a.nz; }
 
 template <int MODEL, int ST>
 hipError_t step_ms(bool glob, const StepArgs& a, int block, hipStream_t s) {
     dim3 grid(step_blocks(a, glob, block)), blk(block);
     if (!glob && a.mode == 3) {
-        if constexpr (tb_model<MODEL>) {
-            if (a.tb_k < 2 || 2 * a.tb_k >= TB_TX || 2 * a.tb_k >= TB_TY || a.nz != 1) return hipErrorInvalidValue;
-            StepArgs b = a;
-            b.tb_bx = (a.nx + TB_TX - 2 * a.tb_k - 1) / (TB_TX - 2 * a.tb_k);
-            const int by = (a.ny + TB_TY - 2 * a.tb_k - 1) / (TB_TY - 2 * a.tb_k);
-            hipLaunchKernelGGL((k_step_tb<MODEL, ST, TB_TX, TB_TY>), dim3(b.tb_bx * by), dim3(TB_TX * TB_TY), 0, s, b);
-            return hipGetLastError();
-        } else {
-            return hipErrorInvalidValue;
-        }
+        if constexpr (tb_model<MODEL>) return blocked2d_ms<MODEL, ST>(a, s);
+        else return hipErrorInvalidValue;
     } else if (!glob && a.mode == 1) {
         hipLaunchKernelGGL((k_step_bulk<MODEL, ST, step_waves<MODEL, ST>()>), grid, blk, 0, s, a);
     } else if (!glob && a.mode == 2) {
@@ -2754,6 +2644,8 @@ hipError_t batch_m(int st, bool glob, const BatchCase* cases, const int2* tiles,
 #define TCLBX_FAM(name) name##_all
 #endif
 hipError_t step_2d_f64(int model, int storage, bool globals, const StepArgs& a, int block, hipStream_t s);
+hipError_t blocked_batch_2d_f64(int model, int storage, const BatchCase* cases, const int2* items, int nitems,
+                                int phase, int steps, const BlockedBatch& b, hipStream_t s);
 hipError_t init_2d_f64(int model, int storage, const StepArgs& a, int block, hipStream_t s);
 hipError_t batch_2d_f64(int model, int storage, bool globals, const BatchCase* cases, const int2* tiles, int ntiles,
                     int phase, double* gpart, int grid, int block, hipStream_t s);
@@ -2784,6 +2676,8 @@ hipError_t batch_cumavg_f64(int model, int storage, bool globals, const BatchCas
 hipError_t quantity_cumavg_f64(int model, int storage, int q, const StepArgs& a, int x0, int y0, int z0, int rx, int ry,
                        int rz, double scale, double* out, hipStream_t s);
 hipError_t step_2d_f32(int model, int storage, bool globals, const StepArgs& a, int block, hipStream_t s);
+hipError_t blocked_batch_2d_f32(int model, int storage, const BatchCase* cases, const int2* items, int nitems,
+                                int phase, int steps, const BlockedBatch& b, hipStream_t s);
 hipError_t init_2d_f32(int model, int storage, const StepArgs& a, int block, hipStream_t s);
 hipError_t batch_2d_f32(int model, int storage, bool globals, const BatchCase* cases, const int2* tiles, int ntiles,
                     int phase, double* gpart, int grid, int block, hipStream_t s);

@@ -110,10 +110,10 @@ Lattice::Lattice(const ModelDef* m, int nx_, int ny_, int nz_, int storage_)
     if (!coll) coll = m->nodetype("BGK");
     bulk_val_ = coll ? coll->value : 0u;
     if (const char* e = std::getenv("TCLBX_SORTED_DISPATCH")) sorted_ = std::atoi(e) != 0 && coll != nullptr;
-    tb_auto_ = temporal_blocking_model(m->id);
+    tb_auto_ = blocked2d_model(m->id);
     if (const char* e = std::getenv("TCLBX_TEMPORAL_BLOCKING"))
         if (tb_auto_ && std::atoi(e) >= 0) {
-            tb_k_ = std::min(TB_TILE / 2 - 1, std::atoi(e));
+            tb_k_ = std::min(TB_MAX_K, std::atoi(e));
             tb_auto_ = false;
         }
     hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
@@ -310,15 +310,11 @@ void Lattice::set_stochastic_rounding(bool on, unsigned seed) {
     drop_graph();
 }
 
-bool temporal_blocking_model(int id) {
-    return id == MODEL_D2Q9_SRT || id == MODEL_D2Q9_SRT_DRAG || id == MODEL_D2Q9 || id == MODEL_D2Q9_DRAG;
-}
-
 void Lattice::set_temporal_blocking(int k) {
-    if (k < -1 || k > TB_TILE / 2 - 1)
-        throw std::invalid_argument("temporal blocking takes -1 (timed) or 0-" + std::to_string(TB_TILE / 2 - 1) +
-                                    " steps per launch");
-    if ((k > 1 || k == -1) && !temporal_blocking_model(model->id))
+    if (k < -1 || k > TB_MAX_K)
+        throw std::invalid_argument("temporal blocking takes -1 (by the lattice's size) or 0-" +
+                                    std::to_string(TB_MAX_K) + " steps per launch");
+    if ((k > 1 || k == -1) && !blocked2d_model(model->id))
         throw std::invalid_argument("temporal blocking applies to d2q9_SRT, d2q9_SRT_drag, d2q9 and d2q9_drag, not " +
                                     model->name);
     tb_auto_ = k == -1;
@@ -326,64 +322,24 @@ void Lattice::set_temporal_blocking(int k) {
     drop_graph();
 }
 
-// Chooses the temporal blocking by timing real steps: the plain steps
-// [i, i + 270) of the current Iterate run in three rounds of 30 steps per
-// candidate (single steps, 3 and 5 per launch), each candidate's best
-// round counting, and the fastest per step is kept; returns the index of
-// the next step.  Every candidate gives the same bits, so the steps count
-// as the run's own.  (Trial steps that leave the state as it is, reading
-// one snapshot over and over, keep their input in the L2 and time the
-// single step at two thirds of its real cost on small lattices.)  Blocking
-// wins where a lattice is too small for one step to fill the GPU or its
-// snapshots sit in the Infinity Cache, and loses on lattices whose steps
-// stream from HBM (the halo is computed again, at lower occupancy); which
-// k is best depends on the storage format (the FP64 tile allows one block
-// per CU) and on how the tiles divide over the CUs.
-int Lattice::tune_blocking(int i) {
+const Blocking& Lattice::blocking(int k) {
+    if (tb_split_.empty()) tb_split_.resize(TB_MAX_K + 1);
+    if (tb_split_[k].k != k) tb_split_[k] = blocking2d(nx, ny, storage, k);
+    return tb_split_[k];
+}
+
+// the number of steps per launch of a lattice left to choose it
+void Lattice::choose_blocking() {
+    if (!tb_auto_) return;
     tb_auto_ = false;
-    struct Events {
-        hipEvent_t e[2] = {nullptr, nullptr};
-        ~Events() {
-            for (hipEvent_t x : e)
-                if (x) (void)hipEventDestroy(x);
-        }
-    } ev;
-    hip_check(hipEventCreate(&ev.e[0]), "event create");
-    hip_check(hipEventCreate(&ev.e[1]), "event create");
-    const int ks[3] = {0, 3, 5};
-    float best[3] = {0, 0, 0};
-    for (int round = 0; round < TB_TUNE_ROUNDS; round++) {
-        for (int c = 0; c < 3; c++) {
-            const int k = ks[c];
-            tb_k_ = k;
-            hip_check(hipEventRecord(ev.e[0], stream_), "event record");
-            for (int done = 0; done < TB_TUNE_SAMPLE;) {
-                if (k > 1)
-                    launch_blocked(snap_, 1 - snap_, iter_ + i);
-                else
-                    launch(snap_, 1 - snap_, false, iter_ + i);
-                snap_ = 1 - snap_;
-                i += k > 1 ? k : 1;
-                done += k > 1 ? k : 1;
-            }
-            hip_check(hipEventRecord(ev.e[1], stream_), "event record");
-            hip_check(hipEventSynchronize(ev.e[1]), "tune blocking");
-            float ms = 0;
-            hip_check(hipEventElapsedTime(&ms, ev.e[0], ev.e[1]), "event elapsed");
-            const float per_step = ms / (float)TB_TUNE_SAMPLE;
-            if (round == 0 || per_step < best[c]) best[c] = per_step;
-        }
-    }
-    int bi = 0;
-    for (int c = 1; c < 3; c++)
-        if (best[c] < best[bi]) bi = c;
-    tb_k_ = ks[bi];
+    const Blocking b = blocking2d(nx, ny, storage, 0);
+    tb_k_ = b.k;
     if (const char* e = std::getenv("TCLBX_TUNE_LOG"); e && std::atoi(e) != 0)
-        std::fprintf(stderr, "tclbx: %s %dx%d %s, us per step: single %.3f, 3 per launch %.3f, 5 per launch %.3f -> %d\n",
-                     model->name.c_str(), nx, ny, storage_name(storage), 1e3 * best[0], 1e3 * best[1], 1e3 * best[2],
-                     tb_k_);
+        std::fprintf(stderr, "tclbx: %s %dx%d %s: %d steps per launch, %s\n", model->name.c_str(), nx, ny,
+                     storage_name(storage), b.k,
+                     b.rows ? ("waves of " + std::to_string(b.rows) + " rows").c_str()
+                            : ("tiles of " + std::to_string(b.tx) + "x" + std::to_string(b.ty)).c_str());
     drop_graph();
-    return i;
 }
 
 // steps of one replay of the captured loop: graph_steps_, or with temporal
@@ -394,12 +350,21 @@ int Lattice::graph_len() const {
     return std::max(2, (graph_steps_ / k) & ~1) * k;
 }
 
-// blocked_k() plain steps in one launch, snapshot `from` -> `to`; the first
-// computes iteration `step` (the key of stochastic rounding)
-void Lattice::launch_blocked(int from, int to, int step) {
-    StepArgs a = args(from, to, false);
+void Lattice::set_blocking(StepArgs& a, int k) {
+    const Blocking& b = blocking(k);
     a.mode = 3;
-    a.tb_k = tb_k_;
+    a.tb_k = k;
+    a.tb_rows = b.rows;
+    a.tb_tx = b.tx;
+    a.tb_ty = b.ty;
+    a.tb_nt = b.nt;
+}
+
+// k plain steps in one launch, snapshot `from` -> `to`; the first computes
+// iteration `step` (the key of stochastic rounding)
+void Lattice::launch_blocked(int k, int from, int to, int step) {
+    StepArgs a = args(from, to, false);
+    set_blocking(a, k);
     a.sr_step = (unsigned)step;
     a.sr_seed = sr_seed_;
     hip_check(launch_step(model->id, storage, false, a, block_, stream_), "temporally blocked step");
@@ -540,8 +505,7 @@ void Lattice::run_graph_steps(int nsteps) {
             StepArgs a = args(i % 2, (i + 1) % 2, false);
             hipError_t e = hipSuccess;
             if (k > 1) {
-                a.mode = 3;
-                a.tb_k = k;
+                set_blocking(a, k);
                 e = launch_step(model->id, storage, false, a, block_, stream_);
             } else if (sorted_) {
                 a.mode = 1;
@@ -625,7 +589,8 @@ void Lattice::tune_rows() {
 void Lattice::Prepare() {
     upload_zone();
     ensure_list();
-    if (tune_rpt_ && N >= (1u << 20)) tune_rows();
+    choose_blocking();
+    if (tune_rpt_ && blocked_k() == 1 && N >= (1u << 20)) tune_rows();
     if (graph_steps_ >= 2 && !sr_) {
         run_graph_steps(0);  // capture only
         hip_check(hipStreamSynchronize(stream_), "Prepare");
@@ -636,31 +601,29 @@ void Lattice::Iterate(int niter, int iter_type) {
     if (niter < 0) throw std::invalid_argument("negative iteration count");
     upload_zone();
     ensure_list();
-    // lattices large enough for the tiling to matter are tuned once, on
-    // the first Iterate that runs enough steps to repay the trial launches
-    // (or earlier, by Prepare)
-    if (tune_rpt_ && niter >= 16 && N >= (1u << 20)) tune_rows();
     int last_glob = iter_type & ITER_LASTGLOB;
     if (iter_type & ITER_INTEG) last_glob = 0;
     const bool every_glob = (iter_type & ITER_GLOBS) != 0;
+    const int plain_end = niter - (last_glob ? 1 : 0);
+    if (!every_glob && plain_end >= 2) choose_blocking();
+    const int k = every_glob ? 1 : blocked_k();
+    // lattices large enough for the tiling to matter are tuned once, on
+    // the first Iterate that runs enough steps to repay the trial launches
+    // (or earlier, by Prepare); blocked steps have no rows per tile
+    if (tune_rpt_ && k == 1 && niter >= 16 && N >= (1u << 20)) tune_rows();
     hip_check(hipEventRecord(ev0_, stream_), "event record");
     int i = 0;
     // leading plain steps until snapshot 0 is current, then whole graph
     // replays, then the tail (the Globals step is always launched directly);
     // a loop not yet captured is captured only when it will be replayed at
     // least twice
-    const int plain_end = niter - (last_glob ? 1 : 0);
-    // the first Iterate with enough plain steps times the temporal blocking
-    // on them
-    if (blocking_to_tune() && !every_glob && plain_end >= TB_TUNE_STEPS) i = tune_blocking(i);
     const bool captured = graph_exec_ != nullptr && graph_version_ == params_version_;
-    const int k = every_glob ? 1 : blocked_k();
     const int lead = snap_ != 0 ? k : 0;
     const int glen = graph_len();
-    if (!every_glob && !sr_ && graph_steps_ >= 2 && plain_end - i - lead >= (captured ? 1 : 2) * glen) {
+    if (!every_glob && !sr_ && graph_steps_ >= 2 && plain_end - lead >= (captured ? 1 : 2) * glen) {
         if (snap_ != 0) {
             if (k > 1)
-                launch_blocked(snap_, 1 - snap_, iter_ + i);
+                launch_blocked(k, snap_, 1 - snap_, iter_ + i);
             else
                 launch(snap_, 1 - snap_, false, iter_ + i);
             snap_ = 1 - snap_;
@@ -672,10 +635,13 @@ void Lattice::Iterate(int niter, int iter_type) {
             i += reps * glen;
         }
     }
-    // the remaining plain steps: blocked launches while k are left
-    for (; k > 1 && plain_end - i >= k; i += k) {
-        launch_blocked(snap_, 1 - snap_, iter_ + i);
+    // the remaining plain steps, spread evenly over blocked launches of at
+    // most k steps (a last single step launches below)
+    while (k > 1 && plain_end - i >= 2) {
+        const int left = plain_end - i, launches = (left + k - 1) / k, kk = (left + launches - 1) / launches;
+        launch_blocked(kk, snap_, 1 - snap_, iter_ + i);
         snap_ = 1 - snap_;
+        i += kk;
     }
     for (; i < niter; i++) {
         const bool glob = every_glob || (last_glob && i == niter - 1);

@@ -104,12 +104,11 @@ public:
     void set_stochastic_rounding(bool on, unsigned seed);
     bool stochastic_rounding() const { return sr_; }
     // temporal blocking of the plain steps of the 2D models d2q9_SRT,
-    // d2q9_SRT_drag, d2q9 and d2q9_drag: k (2 to TB_TILE/2 - 1) steps per
-    // launch on tiles held in LDS, bit-identical to k single steps; 0 or 1:
-    // off; -1 (the default of these models): chosen on lattices under 2^23
-    // nodes by timing the first 270 plain steps of the first Iterate that
-    // runs that many (tune_blocking).  Steps with Globals take the single
-    // step.
+    // d2q9_SRT_drag, d2q9 and d2q9_drag: up to k (2 to TB_MAX_K) steps per
+    // launch, bit-identical to single steps; 0 or 1: off; -1 (the default
+    // of these models): chosen by the lattice's size and storage format
+    // (blocking2d) when it first iterates.  Steps with Globals take the
+    // single step.
     void set_temporal_blocking(int k);
     int temporal_blocking() const { return tb_k_; }
 
@@ -122,16 +121,14 @@ private:
     StepArgs args(int from, int to, bool glob) const;
     void upload_zone();
     void launch(int from, int to, bool glob, int step = 0);
-    void launch_blocked(int from, int to, int step = 0);
+    void launch_blocked(int k, int from, int to, int step);
+    const Blocking& blocking(int k);
+    void set_blocking(StepArgs& a, int k);
+    void choose_blocking();
     int blocked_k() const { return tb_k_ > 1 ? tb_k_ : 1; }
     int graph_len() const;
     void drop_graph();
     void tune_rows();
-    int tune_blocking(int i);
-    // the timing of the temporal blocking: rounds x 3 candidates x steps
-    static constexpr int TB_TUNE_ROUNDS = 3, TB_TUNE_SAMPLE = 30;
-    static constexpr int TB_TUNE_STEPS = TB_TUNE_ROUNDS * 3 * TB_TUNE_SAMPLE;
-    bool blocking_to_tune() const { return tb_auto_ && N < (1u << 23); }
     void run_graph_steps(int nsteps);
     void ensure_list();
 
@@ -171,10 +168,9 @@ private:
     unsigned sr_seed_ = 0;
     int tb_k_ = 0;
     bool tb_auto_ = false;
+    std::vector<Blocking> tb_split_;  // the split of k steps per launch, by k, as needed
 };
 
-// the models the temporally blocked step covers
-bool temporal_blocking_model(int model_id);
 // hipError_t -> exception with a message naming the call
 void hip_check(hipError_t e, const char* what);
 // steps per captured graph of a new Lattice or Batch: 32, or the

@@ -3,10 +3,9 @@ Drag and Lift) stepped in one storage format.
 
     python -m tclb_amd.cylinder --steps 8192 --storage f64 [--temporal-blocking K]
 
-With --temporal-blocking K the plain steps run K per launch on LDS tiles
-(bit-identical to single steps; 0: single steps; -1, the default: the
-lattice times 1, 3 and 5 per launch on the first 270 warm-up steps and
-keeps the fastest).  `prepare()` (rows-per-tile timing, graph capture) and
+With --temporal-blocking K the plain steps run K per launch (bit-identical
+to single steps; 0: single steps; -1, the default: the number its size and
+storage format call for).  `prepare()` (rows-per-tile timing, graph capture) and
 512 warm-up steps, then `steps` timed steps: wall-clock and HIP-event microseconds per step,
 MLUPS, and the Drag and Lift of a final Globals step.  The environment
 variable TCLBX_GRAPH_STEPS sets the length of the captured step loops (0:

@@ -6,9 +6,8 @@
 Every node of an n^3 (2D models: n^2) periodic box carries the model's
 collision NodeType and nothing else, so each step is the plain pull +
 collision of every node; a small body force keeps the flow moving.  For
-each model and storage format: `warmup` steps (2D models: at least 300,
-whose first 270 time the choice of the temporal blocking, reported as
-`temporal_blocking`), then `steps` timed steps
+each model and storage format: `warmup` steps (the steps per launch the
+2D models chose are reported as `temporal_blocking`), then `steps` timed steps
 (HIP events around the step launches), MLUPS and the algorithmic HBM
 bytes per node step (read and write Q stored values, the 2-byte NodeType,
 the FP64 averages of the AVG builds read and written in place, the FP64
@@ -55,9 +54,7 @@ def run(model, fmt, n, steps, warmup, shape=None):
             lat.set_setting(k, v)
         lat.init()
         lat.prepare()
-        # the 2D lattices time their temporal blocking on the first 270
-        # steps of an Iterate: those stay in the warm-up
-        lat.iterate(max(warmup, 300) if m.Q == 9 else warmup)
+        lat.iterate(warmup)
         lat.iterate(steps)
         ms, _ = lat.timing()
         nodes = nx * ny * nz

@@ -1,0 +1,71 @@
+"""The blocked steps (several plain steps per launch) give the single steps'
+bits at the sizes where they can go wrong: strips and tiles that end inside
+the lattice, segments of uneven length, lattices narrower than a strip."""
+import numpy as np
+import pytest
+
+import tclb_amd
+from tclb_amd import ITER_NORM
+
+from test_gpu_parity import random_case, say
+
+pytestmark = pytest.mark.gpu
+
+
+def same(a, b):
+    return np.array_equal(a, b, equal_nan=True)
+
+
+@pytest.mark.parametrize("model,storage,nx,ny,k", [
+    ("d2q9_SRT", "f64", 1031, 1021, 2),         # 1,031 = 16 strips of 62 and 39 columns
+    ("d2q9_drag", "f64", 1031, 1021, 4),
+    ("d2q9_SRT_drag", "f64", 57, 18500, 5),     # narrower than a strip of 56: its halo wraps onto itself
+    ("d2q9", "f16s", 2053, 2049, 3),
+    ("d2q9_SRT", "f32s", 70001, 61, 5),         # rows that a segment of 12 does not divide
+])
+def test_marching_waves_are_bit_identical(model, storage, nx, ny, k):
+    """Lattices past the line where k <= 5 steps per launch march, against
+    single steps: a whole launch, a shorter rest of steps, stochastic
+    rounding in the 16-bit format."""
+    say(f"marching waves {model} {storage} {nx}x{ny} k={k}")
+    case = random_case(model, nx, ny, 1, seed=7)
+    a, b = case.build(storage), case.build(storage)
+    if storage == "f16s":
+        for lat in (a, b):
+            lat.set_stochastic_rounding(True, seed=3)
+    a.temporal_blocking, b.temporal_blocking = k, 0
+    for n in (k, 2 * k - 1):
+        a.iterate(n, ITER_NORM)
+        b.iterate(n, ITER_NORM)
+        fa = a.get_f()
+        if n == k:
+            assert np.mean(np.isfinite(fa)) > 0.5
+        assert same(fa, b.get_f()), n
+
+
+@pytest.mark.parametrize("storage,sizes", [
+    ("f64", [(700, 601), (61, 500), (901, 800)]),   # marching waves
+    ("f64", [(75, 41), (20, 9), (130, 70)]),        # tiles, one case smaller than a tile
+    ("f16s", [(75, 41), (20, 9), (130, 70)]),
+])
+def test_blocked_batch_steps_are_bit_identical(storage, sizes):
+    """Every case of a batch steps as a lone lattice's single steps, through
+    whole launches, rests, graph replays and a case that joins mid-run."""
+    say(f"blocked batch {storage} {sizes}")
+    cases = [random_case("d2q9_drag", nx, ny, 1, seed=11 + i) for i, (nx, ny) in enumerate(sizes)]
+    batch = tclb_amd.Batch("d2q9_drag", storage, 1 << 30)
+    lats = []
+    for c in cases:
+        lat = c.build(storage)
+        lat.temporal_blocking = 0
+        lats.append(lat)
+    ids = [batch.add(c) for c in cases[:2]]
+    batch.set_graph_steps(2)
+    for step, n in enumerate((1, 7, 24)):
+        if step == 1:
+            ids.append(batch.add(cases[2]))
+        batch.iterate(n)
+        for i, lat in zip(ids, lats):
+            lat.iterate(n)
+            assert same(batch.get_f(i), lat.get_f()), (n, i)
+            assert same(batch.globals(i), lat.globals), (n, i)
