@@ -232,17 +232,15 @@ StepArgs Batch::case_args(const Case& c) const {
     a.zone = c.d_zone;
     a.pitch = (long long)c.pitch;
     a.nx = c.nx; a.ny = c.ny; a.nz = c.nz;
-    a.flat = tune_.flat;
+    // flat runs for every step (a tuning that asks for them), or by default
+    // for the plain steps of the cases whose rows leave lanes idle
+    a.flat = tune_.flat ? 3 : (tune_auto_ && flat_pays(c.nx) ? 1 : 0);
     a.inv_nx = 1.0 / c.nx;
     a.inv_ny = 1.0 / c.ny;
-    if (tune_.flat) {
-        // a "row" of a flat tile is a run of `block` consecutive nodes
-        a.bpr = 1;
-        a.rpb = globals_rows_per_block(((long long)c.N + tune_.block - 1) / tune_.block, 1);
-    } else {
-        a.bpr = (c.nx + tune_.block - 1) / tune_.block;
-        a.rpb = globals_rows_per_block(c.ny * c.nz, a.bpr);
-    }
+    a.bpr = (c.nx + tune_.block - 1) / tune_.block;
+    // a "row" of a flat tile is a run of `block` consecutive nodes
+    a.rpb = tune_.flat ? globals_rows_per_block(((long long)c.N + tune_.block - 1) / tune_.block, 1)
+                       : globals_rows_per_block(c.ny * c.nz, a.bpr);
     a.rpt = tune_.rpt;
     a.zcols = (int)model->zonal.size();
     a.nzones = model->zone_max + 1;
@@ -577,6 +575,13 @@ void Batch::SetTuning(const Tuning& t) {
     if (t.grid < 0) throw std::invalid_argument("grid must be >= 0");
     if (t.order != 0 && t.order != 1) throw std::invalid_argument("tile order must be 0 or 1");
     tune_ = t;
+    tune_auto_ = false;
+    dirty_ = true;
+}
+
+void Batch::SetTileOrder(int order) {
+    if (order != 0 && order != 1) throw std::invalid_argument("tile order must be 0 or 1");
+    tune_.order = order;
     dirty_ = true;
 }
 
@@ -587,6 +592,7 @@ Tuning Batch::Autotune(int steps) {
     if (steps < 1) throw std::invalid_argument("autotune needs at least one step");
     if (active_.empty()) return tune_;
     const Tuning saved = tune_;
+    tune_auto_ = false;
     trials_.clear();
     Tuning best = saved;
     best.us_per_step = 1e300;

@@ -90,6 +90,7 @@ public:
     // keep the fastest
     Tuning Autotune(int steps);
     void SetTuning(const Tuning& t);
+    void SetTileOrder(int order);
     // stochastic rounding of every case's stores (16-bit formats only); a
     // case is keyed by its own node index, iteration and `seed`, as a lone
     // Lattice with the same seed keys it, so its result is the same alone and
@@ -160,6 +161,7 @@ private:
     // plain steps per launch of a 2D batch: tb_k_ = 0 by size, else fixed (1:
     // single steps); blocked_ is what the current set of cases got
     int tb_k_ = 0;
+    bool tune_auto_ = true;  // no tuning was set or timed
     BlockedBatch blocked_;
     std::vector<int> order_;  // case id of device slot i
     hipStream_t stream_ = nullptr;

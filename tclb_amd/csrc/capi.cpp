@@ -553,11 +553,7 @@ int tclbx_batch_set_tuning(tclbx_batch* b, int flat, int block, int rows_per_til
 int tclbx_batch_tile_order(tclbx_batch* b, int set, int* order) {
     CHECK_B(b);
     return guard([&]() {
-        if (set >= 0) {
-            Tuning t = b->b->tuning();
-            t.order = set;
-            b->b->SetTuning(t);
-        }
+        if (set >= 0) b->b->SetTileOrder(set);
         if (order) *order = b->b->tuning().order;
         return TCLBX_OK;
     });

@@ -37,7 +37,8 @@ struct StepArgs {
     int bpr;               // blocks per (y,z) row
     int rpb;               // rows walked by one block of a Globals step
     int rpt;               // rows walked by one block of a plain step
-    int flat;              // 1: tiles are runs of the linear node index, not row segments
+    int flat;              // tiles are runs of the linear node index, not row segments: bit 0
+                           // for plain steps, bit 1 for Globals steps
     double inv_nx;         // 1/nx (flat tiles: node index -> row)
     double inv_ny;         // 1/ny (flat tiles: row -> y, z)
     int zcols, nzones;

@@ -241,7 +241,7 @@ hipError_t launch_blocked_batch(int model, int storage, const BatchCase* cases, 
 
 int step_blocks(const StepArgs& a, bool globals, int block) {
     const int rpb = globals ? a.rpb : a.rpt;
-    if (a.flat) {
+    if (a.flat & (globals ? 2 : 1)) {
         const long long chunks = ((long long)a.nx * a.ny * a.nz + block - 1) / block;
         return (int)((chunks + rpb - 1) / rpb);
     }

@@ -2108,7 +2108,7 @@ __device__ __forceinline__ void split_node(unsigned n, int nx, double inv_nx, in
 template <int MODEL, int ST, bool GLOB, int DISPATCH = 0>
 __device__ __forceinline__ void step_tile(const StepArgs& a, int tile, int rpb, int slot, int nslots) {
     using L = Lat<MODEL>;
-    if (a.flat) {
+    if (a.flat & (GLOB ? 2 : 1)) {
         // runs of blockDim consecutive nodes (rows of the lattice are
         // concatenated, no lane is left idle at the end of a row)
         double g[L::G > 0 ? L::G : 1];

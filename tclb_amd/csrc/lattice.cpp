@@ -32,6 +32,15 @@ int pick_block(int nx) {
 }
 }  // namespace
 
+// A plain step walks runs of 256 consecutive nodes instead of row segments
+// where a row is no multiple of 256 nodes: no lane idles at a row's end, and
+// a small lattice's blocks are all full.  us per step, best row segments
+// against runs of 256: d3q19 f64 157x131x97 151 / 114, 96^3 54.8 / 53.8, f16s
+// 71x150x100 29.8 / 17.8, 160x159x155 66.9 / 55.5; d3q27 f32 129x97x113 98.3 /
+// 68.3; d3q27_cumulant f16s 160x128x96 65.8 / 53.7; at 256^3 the two are equal
+// (f16s 235.7 / 235.1).
+bool flat_pays(int nx) { return nx % 256 != 0; }
+
 int default_graph_steps() {
     // a captured loop starts and ends on snapshot 0, so its length is even:
     // an odd value is rounded down (1 -> 0, no graph)
@@ -99,6 +108,7 @@ Lattice::Lattice(const ModelDef* m, int nx_, int ny_, int nz_, int storage_)
     }
     hip_check(hipMalloc((void**)&d_zone_, std::max<size_t>(1, zone_.size()) * sizeof(double)), "hipMalloc(zone)");
     set_block(pick_block(nx));
+    flat_ = flat_pays(nx);
     const int G = kernel_nglobals(m->id);
     hip_check(hipMalloc((void**)&d_glob_, MAX_GLOBALS * sizeof(double)), "hipMalloc(globals)");
     hip_check(hipMemsetAsync(d_glob_, 0, MAX_GLOBALS * sizeof(double), stream_), "hipMemset(globals)");
@@ -139,6 +149,7 @@ Lattice::~Lattice() {
 void Lattice::set_block(int b) {
     if (b != 64 && b != 128 && b != 256) throw std::invalid_argument("block must be 64, 128 or 256");
     block_ = b;
+    flat_ = false;   // a block that the caller sets is a row segment's
     bpr_ = (nx + b - 1) / b;
     nblocks_ = bpr_ * ny * nz;
     rpb_ = globals_rows_per_block((long long)ny * nz, bpr_);
@@ -283,7 +294,7 @@ StepArgs Lattice::args(int from, int to, bool glob) const {
     a.bpr = bpr_;
     a.rpb = rpb_;
     a.rpt = rpt_;
-    a.flat = 0;
+    a.flat = !glob && flat_ ? 1 : 0;
     a.inv_nx = 1.0 / nx;
     a.inv_ny = 1.0 / ny;
     a.zcols = zcols_;
@@ -474,12 +485,12 @@ void Lattice::launch(int from, int to, bool glob, int step) {
     a.sr_key = sr_key((unsigned)step, sr_seed_);
     if (sorted_ && !glob) {
         a.mode = 1;
-        hip_check(launch_step(model->id, storage, false, a, block_, stream_), "step kernel (bulk)");
+        hip_check(launch_step(model->id, storage, false, a, plain_block(), stream_), "step kernel (bulk)");
         a.mode = 2;
-        hip_check(launch_step(model->id, storage, false, a, block_, stream_), "step kernel (sorted list)");
+        hip_check(launch_step(model->id, storage, false, a, plain_block(), stream_), "step kernel (sorted list)");
         return;
     }
-    hip_check(launch_step(model->id, storage, glob, a, block_, stream_), "step kernel");
+    hip_check(launch_step(model->id, storage, glob, a, glob ? block_ : plain_block(), stream_), "step kernel");
     if (glob) {
         hip_check(launch_reduce_globals(d_gpart_, step_blocks(a, true, block_), kernel_nglobals(model->id),
                                         model->sum_globals, d_glob_, stream_), "globals reduction");
@@ -509,11 +520,11 @@ void Lattice::run_graph_steps(int nsteps) {
                 e = launch_step(model->id, storage, false, a, block_, stream_);
             } else if (sorted_) {
                 a.mode = 1;
-                e = launch_step(model->id, storage, false, a, block_, stream_);
+                e = launch_step(model->id, storage, false, a, plain_block(), stream_);
                 a.mode = 2;
-                if (e == hipSuccess) e = launch_step(model->id, storage, false, a, block_, stream_);
+                if (e == hipSuccess) e = launch_step(model->id, storage, false, a, plain_block(), stream_);
             } else {
-                e = launch_step(model->id, storage, false, a, block_, stream_);
+                e = launch_step(model->id, storage, false, a, plain_block(), stream_);
             }
             if (e != hipSuccess) {
                 hipGraph_t g = nullptr;

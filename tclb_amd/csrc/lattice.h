@@ -147,6 +147,8 @@ private:
     double* d_glob_ = nullptr;
     std::vector<double> globals_;
     int nblocks_ = 0, block_ = 256, bpr_ = 1, rpb_ = 1;
+    bool flat_ = false;  // plain steps walk runs of the linear index
+    int plain_block() const { return flat_ ? 256 : block_; }
     hipStream_t stream_ = nullptr;
     hipEvent_t ev0_ = nullptr, ev1_ = nullptr;
     double last_ms_ = 0, kernel_ms_ = 0;
@@ -173,6 +175,8 @@ private:
 
 // hipError_t -> exception with a message naming the call
 void hip_check(hipError_t e, const char* what);
+// whether plain steps of rows of nx nodes walk runs of the linear index
+bool flat_pays(int nx);
 // steps per captured graph of a new Lattice or Batch: 32, or the
 // environment's TCLBX_GRAPH_STEPS rounded down to an even count (0 or 1:
 // every step launched directly, for tools that do not follow graph launches)

@@ -69,3 +69,25 @@ def test_blocked_batch_steps_are_bit_identical(storage, sizes):
             lat.iterate(n)
             assert same(batch.get_f(i), lat.get_f()), (n, i)
             assert same(batch.globals(i), lat.globals), (n, i)
+
+
+@pytest.mark.parametrize("model,storage,shape", [
+    ("d3q19", "f16s", (71, 15, 10)),          # 10,650 nodes: the last run of 256 is part full
+    ("d3q27", "f32", (129, 7, 6)),
+    ("d3q27_cumulant", "f64", (1, 300, 2)),   # rows of one node
+    ("d2q9_autosym2", "f32s", (255, 9, 1)),
+])
+def test_plain_steps_on_runs_of_the_linear_index(model, storage, shape):
+    """Plain steps on runs of 256 consecutive nodes (the default where rows
+    are no multiple of 256) against row segments, alone and in a batch."""
+    say(f"flat plain steps {model} {storage} {shape}")
+    case = random_case(model, *shape, seed=9)
+    a, b = case.build(storage), case.build(storage)
+    b.set_block(64)
+    batch = tclb_amd.Batch(model, storage, 1 << 26)
+    cid = batch.add(case)
+    for n in (1, 6):
+        for x in (a, b, batch):
+            x.iterate(n)
+        assert same(a.get_f(), b.get_f()) and same(batch.get_f(cid), b.get_f())
+        assert same(a.globals, b.globals) and same(batch.globals(cid), b.globals)
