@@ -238,9 +238,12 @@ int tclbx_set_stochastic_rounding(tclbx_lattice* h, int on, unsigned seed);
  * models, takes the steps per launch that the lattice's size and storage
  * format call for when it first iterates.  Results are those of single
  * steps, bit for bit, stochastic rounding included.  Steps with Globals take
- * the single step.  Batches of these models step the same way.  The
- * environment's TCLBX_TEMPORAL_BLOCKING=k (k >= 0) fixes it for new
- * lattices and batches.  No counterpart in the reference, which launches
+ * the single step.  Batches of these models step the same way.  Lattices of
+ * the 3D models take two steps per launch, bit for bit those of single steps,
+ * where their model, storage format and size make that faster; 0 or 1 turns
+ * that off too (-1 and larger numbers are refused).  The environment's
+ * TCLBX_TEMPORAL_BLOCKING=k (k >= 0; 2 and more for the 2D models only)
+ * fixes it for new lattices and batches.  No counterpart in the reference, which launches
  * one kernel per iteration (src/Lattice.cu.Rt:1246-1297). */
 int tclbx_set_temporal_blocking(tclbx_lattice* h, int steps);
 /* the steps per launch in use (0: single steps, also before the first tclbx_iterate chose) */

@@ -537,11 +537,11 @@ class Lattice:
 
     @property
     def temporal_blocking(self):
-        """Plain steps per launch of the temporally blocked 2D step in use (0:
-        single steps).  Set k >= 2 to fix it, 0 to turn it off, -1 to take
-        the number the lattice's size and storage format call for (the
-        default of d2q9_SRT, d2q9_SRT_drag, d2q9 and d2q9_drag, chosen when
-        the lattice first iterates)."""
+        """Plain steps per launch in use (0: single steps).  Set k >= 2 to
+        fix it, 0 to turn it off, -1 to take the number the lattice's size
+        and storage format call for (the default of d2q9_SRT, d2q9_SRT_drag,
+        d2q9 and d2q9_drag, chosen when the lattice first iterates).  3D
+        lattices choose between one and two by themselves and take only 0."""
         k = ctypes.c_int()
         _check(lib().tclbx_get_temporal_blocking(self._h, ctypes.byref(k)))
         return k.value

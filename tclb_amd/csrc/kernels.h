@@ -48,15 +48,16 @@ struct StepArgs {
     // below the zone) is bulk_val, the plain collision node, so that every
     // wavefront takes the same branch; mode 2 the list[0..list_n) of the
     // other nodes, sorted by class, one thread each.  Mode 3: tb_k plain
-    // steps in one launch of the temporally blocked step (2D models), as
-    // the tb_* fields below say (a Blocking of blocking2d)
+    // steps in one launch of the temporally blocked step, as the tb_* fields
+    // below say (a Blocking of blocking2d or blocking3d)
     int mode;
     unsigned class_mask, bulk_val;
     const unsigned* list;
     unsigned list_n;
     int tb_k;
-    int tb_rows;        // marching waves: rows each wave writes; 0: LDS tiles
-    int tb_tx, tb_ty;   // LDS tiles: nodes along x and y
+    int tb_rows;        // marching waves: rows each wave writes (3D: layers of a
+                        // block); 0: LDS tiles
+    int tb_tx, tb_ty;   // LDS tiles, 3D tiles: nodes along x and y
     int tb_nt;          // LDS tiles: stores past the L2
     // stochastic rounding of the stores of a 16-bit format (0: nearest even);
     // sr_key = sr_key(iteration the step computes, the lattice's seed)
@@ -95,6 +96,9 @@ bool blocked2d_model(int model);
 // The split for a lattice of nx x ny nodes: of k steps per launch, or with k =
 // 0 of the best number of steps (kernels.hip says why the lines lie there).
 Blocking blocking2d(int nx, int ny, int storage, int k);
+// two steps per launch of a 3D lattice: marching tiles (tx x ty columns, rows =
+// layers along z), or k = 1 where single steps are as fast
+Blocking blocking3d(int model, int nx, int ny, int nz, int storage);
 // The same for the lattices of a batch (nx, ny), which share the number of
 // steps, the kind and the block; each lattice's split goes to `cases`.
 struct BlockedBatch {

@@ -222,6 +222,55 @@ BlockedBatch blocking2d_batch(const int2* sizes, int n, int storage, int k, Bloc
     return tile_split(sizes, n, storage, k ? std::vector<int>{k} : std::vector<int>{3, 4, 5}, cases);
 }
 
+// The march's time is rounds of blocks (one per CU: the tile fills its LDS) x
+// (layers + 3 iterations) x the time of an iteration, which depends on the
+// tile and little on the lattice (us, below and above 4M nodes): d3q19 f64
+// 34x15 8.5, 8.9, f32s 66x15 7.1, 7.8, 34x30 7.2, 8.6; FP64 34x10 d3q27 7.5,
+// cumulant 8.8.  So the layers are those of the fewest iterations in all, and
+// the march is taken where they beat the single step's rate (MLUPS, below and
+// above 8M nodes: d3q19 17.3k, 18.1k and 34k, 37.2k, d3q27 12.8k, cumulant
+// 12.5k).  us per step, single / march: d3q19 f64 256^3 924 / 784, 192x176x160
+// 309 / 245, 61x48x57 13.6 / 24 (single stays); f32s 256^3 450 / 352,
+// 192x176x160 156 / 114, 157x131x97 72 / 47; d3q27 f64 256x128x128 326 / 251;
+// cumulant f64 336 / 295.  The 16-bit formats and the 27-velocity float steps
+// are bound by their instructions and gain nothing (d3q19 f16s 256^3 253 /
+// 257, d3q27 f32s 256x128x128 170 / 172).
+Blocking blocking3d(int model, int nx, int ny, int nz, int storage) {
+    struct Tile { int tx, ty; double us, us_large; };
+    const Tile f64[1] = {{34, 15, 8.5, 8.9}}, f32[2] = {{66, 15, 7.1, 7.8}, {34, 30, 7.2, 8.6}};
+    const Tile q27[1] = {{34, 10, 7.5, 7.5}}, cum[1] = {{34, 10, 8.8, 8.8}};
+    const double nodes = (double)nx * ny * nz;
+    const Tile* tiles = nullptr;
+    int ntiles = 1;
+    double mlups = 0;
+    if (model == MODEL_D3Q19 || model == MODEL_D3Q19_LID) {
+        if (storage == ST_F64) { tiles = f64; mlups = nodes < 8e6 ? 17300 : 18100; }
+        if (storage == ST_F32 || storage == ST_F32S) { tiles = f32; ntiles = 2; mlups = nodes < 8e6 ? 34000 : 37200; }
+    } else if (storage == ST_F64 && model == MODEL_D3Q27) {
+        tiles = q27; mlups = 12800;
+    } else if (storage == ST_F64 && (model == MODEL_D3Q27_CUMULANT || model == MODEL_D3Q27_CUMULANT_SMAG)) {
+        tiles = cum; mlups = 12500;
+    }
+    Blocking best;
+    if (!tiles) return best;
+    double best_us = 2 * 0.97 * nodes / mlups;   // two single steps
+    for (int t = 0; t < ntiles; t++) {
+        const int wx = tiles[t].tx - 2, wy = tiles[t].ty - 2;
+        const long long columns = (long long)((nx + wx - 1) / wx) * ((ny + wy - 1) / wy);
+        for (int segs = 1; segs <= nz; segs++) {
+            const int rows = (nz + segs - 1) / segs;
+            const long long blocks = columns * ((nz + rows - 1) / rows);
+            if (blocks > 256 * 64 && segs > 1) break;
+            const double us = (double)((blocks + 255) / 256) * (rows + 3) * (nodes < 4e6 ? tiles[t].us : tiles[t].us_large);
+            if (us < best_us) {
+                best_us = us;
+                best.k = 2; best.rows = rows; best.tx = tiles[t].tx; best.ty = tiles[t].ty;
+            }
+        }
+    }
+    return best;
+}
+
 int blocked2d_items(const StepArgs& a) {
     if (a.tb_rows > 0) return strips2d(a.nx, a.tb_k) * ((a.ny + a.tb_rows - 1) / a.tb_rows);
     const int wx = a.tb_tx - 2 * (a.tb_k - 1), wy = a.tb_ty - 2 * (a.tb_k - 1);

@@ -1,7 +1,7 @@
 // kernels_d3q19.hip -- instantiates and dispatches the node kernels of one
 // family of models (see kernels_impl.h); compiled apart so the families
 // build in parallel.
-#include "kernels_impl.h"
+#include "kernels_march3d.h"
 
 namespace tclbx {
 

@@ -2507,6 +2507,15 @@ template <int MODEL>
 constexpr bool tb_model = MODEL == MODEL_D2Q9_SRT || MODEL == MODEL_D2Q9_SRT_DRAG || MODEL == MODEL_D2Q9 ||
                           MODEL == MODEL_D2Q9_DRAG;
 
+// the same for two steps of a 3D model (kernels_march3d.h, compiled with the 3D
+// families that blocking3d lets take it)
+template <int MODEL, int ST>
+hipError_t blocked3d_ms(const StepArgs& a, hipStream_t s);
+template <int MODEL, int ST>
+constexpr bool march3d_model = (is_d3q19<MODEL> && (ST == ST_F64 || ST == ST_F32 || ST == ST_F32S)) ||
+                               ((MODEL == MODEL_D3Q27 || MODEL == MODEL_D3Q27_CUMULANT ||
+                                 MODEL == MODEL_D3Q27_CUMULANT_SMAG) && ST == ST_F64);
+
 inline int nblocks_of(const StepArgs& a, int block) { return a.bpr * a.ny * a.nz; }
 
 template <int MODEL, int ST>
@@ -2514,6 +2523,7 @@ hipError_t step_ms(bool glob, const StepArgs& a, int block, hipStream_t s) {
     dim3 grid(step_blocks(a, glob, block)), blk(block);
     if (!glob && a.mode == 3) {
         if constexpr (tb_model<MODEL>) return blocked2d_ms<MODEL, ST>(a, s);
+        else if constexpr (march3d_model<MODEL, ST>) return blocked3d_ms<MODEL, ST>(a, s);
         else return hipErrorInvalidValue;
     } else if (!glob && a.mode == 1) {
         hipLaunchKernelGGL((k_step_bulk<MODEL, ST, step_waves<MODEL, ST>()>), grid, blk, 0, s, a);

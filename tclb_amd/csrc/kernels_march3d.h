@@ -188,4 +188,21 @@ hipError_t march3d_ms(const StepArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
+// the tiles that blocking3d may ask for; their written columns, TX - 2, are
+// whole 128-byte lines of a row that starts on one: with a middle of 30 or 62
+// columns, whose rows end inside a line, the stores alone ran at 1.6 TB/s
+// (256^3 f32s, 450 us per single step: 64x16 tiles 494 us, 66x15 352)
+template <int MODEL, int ST>
+hipError_t blocked3d_ms(const StepArgs& a, hipStream_t s) {
+    if constexpr (Lat<MODEL>::Q == 27) {
+        if (a.tb_tx == 34 && a.tb_ty == 10) return march3d_ms<MODEL, ST, 34, 10>(a, s);
+    } else if constexpr (ST == ST_F64) {
+        if (a.tb_tx == 34 && a.tb_ty == 15) return march3d_ms<MODEL, ST, 34, 15>(a, s);
+    } else {
+        if (a.tb_tx == 66 && a.tb_ty == 15) return march3d_ms<MODEL, ST, 66, 15>(a, s);
+        if (a.tb_tx == 34 && a.tb_ty == 30) return march3d_ms<MODEL, ST, 34, 30>(a, s);
+    }
+    return hipErrorInvalidValue;
+}
+
 }  // namespace tclbx

@@ -120,9 +120,10 @@ Lattice::Lattice(const ModelDef* m, int nx_, int ny_, int nz_, int storage_)
     if (!coll) coll = m->nodetype("BGK");
     bulk_val_ = coll ? coll->value : 0u;
     if (const char* e = std::getenv("TCLBX_SORTED_DISPATCH")) sorted_ = std::atoi(e) != 0 && coll != nullptr;
-    tb_auto_ = blocked2d_model(m->id);
+    // (2D: k steps per launch; 3D: two, by size only)
+    tb_auto_ = true;
     if (const char* e = std::getenv("TCLBX_TEMPORAL_BLOCKING"))
-        if (tb_auto_ && std::atoi(e) >= 0) {
+        if (std::atoi(e) >= 0 && (blocked2d_model(m->id) || std::atoi(e) < 2)) {
             tb_k_ = std::min(TB_MAX_K, std::atoi(e));
             tb_auto_ = false;
         }
@@ -343,6 +344,12 @@ const Blocking& Lattice::blocking(int k) {
 void Lattice::choose_blocking() {
     if (!tb_auto_) return;
     tb_auto_ = false;
+    if (!blocked2d_model(model->id)) {
+        tb_split3d_ = blocking3d(model->id, nx, ny, nz, storage);
+        tb_k_ = tb_split3d_.k > 1 ? tb_split3d_.k : 0;
+        drop_graph();
+        return;
+    }
     const Blocking b = blocking2d(nx, ny, storage, 0);
     tb_k_ = b.k;
     if (const char* e = std::getenv("TCLBX_TUNE_LOG"); e && std::atoi(e) != 0)
@@ -362,7 +369,7 @@ int Lattice::graph_len() const {
 }
 
 void Lattice::set_blocking(StepArgs& a, int k) {
-    const Blocking& b = blocking(k);
+    const Blocking& b = model->dim == 2 ? blocking(k) : tb_split3d_;
     a.mode = 3;
     a.tb_k = k;
     a.tb_rows = b.rows;

@@ -108,7 +108,8 @@ public:
     // launch, bit-identical to single steps; 0 or 1: off; -1 (the default
     // of these models): chosen by the lattice's size and storage format
     // (blocking2d) when it first iterates.  Steps with Globals take the
-    // single step.
+    // single step.  3D lattices take two steps per launch where that is
+    // faster (blocking3d); 0 turns that off too, other numbers are refused.
     void set_temporal_blocking(int k);
     int temporal_blocking() const { return tb_k_; }
 
@@ -125,7 +126,9 @@ private:
     const Blocking& blocking(int k);
     void set_blocking(StepArgs& a, int k);
     void choose_blocking();
-    int blocked_k() const { return tb_k_ > 1 ? tb_k_ : 1; }
+    // steps per blocked launch; the sorted dispatch of a 3D lattice, which its
+    // caller asked for, keeps single steps
+    int blocked_k() const { return tb_k_ > 1 && !(sorted_ && model->dim == 3) ? tb_k_ : 1; }
     int graph_len() const;
     void drop_graph();
     void tune_rows();
@@ -170,6 +173,7 @@ private:
     unsigned sr_seed_ = 0;
     int tb_k_ = 0;
     bool tb_auto_ = false;
+    Blocking tb_split3d_;
     std::vector<Blocking> tb_split_;  // the split of k steps per launch, by k, as needed
 };
 

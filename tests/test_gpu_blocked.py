@@ -91,3 +91,33 @@ def test_plain_steps_on_runs_of_the_linear_index(model, storage, shape):
             x.iterate(n)
         assert same(a.get_f(), b.get_f()) and same(batch.get_f(cid), b.get_f())
         assert same(a.globals, b.globals) and same(batch.globals(cid), b.globals)
+
+
+@pytest.mark.parametrize("model,storage,shape", [
+    ("d3q19", "f64", (159, 130, 75)),          # written columns that the lattice ends inside of
+    ("d3q19_lid", "f32s", (157, 131, 60)),     # rows that start inside a memory line
+    ("d3q19", "f32", (256, 91, 64)),
+    ("d3q27", "f64", (128, 60, 130)),
+    ("d3q27_cumulant_SMAG", "f64", (128, 126, 96)),
+])
+def test_marching_tiles_are_bit_identical(model, storage, shape):
+    """3D lattices that take two steps per launch, against single steps: odd
+    and even numbers of plain steps, a change of NodeTypes, the Globals step
+    behind them."""
+    say(f"marching tiles {model} {storage} {shape}")
+    case = random_case(model, *shape, seed=5)
+    a, b = case.build(storage), case.build(storage)
+    b.temporal_blocking = 0
+    for n in (3, 4):
+        a.iterate(n)
+        b.iterate(n)
+        assert a.temporal_blocking == 2 and b.temporal_blocking == 0
+        fa = a.get_f()
+        assert np.mean(np.isfinite(fa)) > 0.5
+        assert same(fa, b.get_f()), n
+        assert same(a.globals, b.globals), n
+        flags = case.flags.copy()
+        v = flags.reshape(-1)
+        v[0:5 * v[1::5].size:5] = v[1::5]
+        a.set_flags(flags)
+        b.set_flags(flags)
