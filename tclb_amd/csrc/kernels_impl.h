@@ -1582,33 +1582,38 @@ __device__ __forceinline__ void cum_inv(R* m) {
 // Dynamics.c.Rt:291-318 are this recursion written out.
 __host__ __device__ constexpr int cum_first_axis(int i) { return i % 3 ? 0 : (i / 3 % 3 ? 1 : 2); }
 
-// term k of the sum for moment i (all indices compile-time constants)
-template <int I, int K>
+// term k of the sum for moment i (all indices compile-time constants); the
+// cumulants of orders above ORDER are zero and their terms left out
+template <int I, int K, int ORDER>
 struct CumTerm {
     static constexpr int j = cum_first_axis(I);
     static constexpr int st = j == 0 ? 1 : (j == 1 ? 3 : 9);
     static constexpr int nx = I % 3 - (j == 0), ny = I / 3 % 3 - (j == 1), nz = I / 9 - (j == 2);
     static constexpr int kx = K % 3, ky = K / 3 % 3, kz = K / 9;
-    static constexpr bool on = kx <= nx && ky <= ny && kz <= nz && !(kx == nx && ky == ny && kz == nz);
+    static constexpr bool on = kx <= nx && ky <= ny && kz <= nz && !(kx == nx && ky == ny && kz == nz) &&
+                               kx + ky + kz + 1 <= ORDER;
     static constexpr int bin = (nx == 2 && kx == 1 ? 2 : 1) * (ny == 2 && ky == 1 ? 2 : 1) * (nz == 2 && kz == 1 ? 2 : 1);
     static constexpr int ck = on ? K + st : 0;
     static constexpr int mk = on ? (nx - kx) + 3 * (ny - ky) + 9 * (nz - kz) : 0;
 };
 
-template <class R, int I, int... K>
+template <class R, int ORDER, int I, int... K>
 __device__ __forceinline__ R cum_sum(const R* c, const R* m, std::integer_sequence<int, K...>) {
     // fused multiply-adds: the float path of this model is arithmetic-bound
     R s = 0;
-    ((CumTerm<I, K>::on
-          ? (void)(s = fma(CumTerm<I, K>::bin == 1 ? c[CumTerm<I, K>::ck] : R(CumTerm<I, K>::bin) * c[CumTerm<I, K>::ck],
-                           m[CumTerm<I, K>::mk], s))
+    ((CumTerm<I, K, ORDER>::on
+          ? (void)(s = fma(CumTerm<I, K, ORDER>::bin == 1 ? c[CumTerm<I, K, ORDER>::ck]
+                                                          : R(CumTerm<I, K, ORDER>::bin) * c[CumTerm<I, K, ORDER>::ck],
+                           m[CumTerm<I, K, ORDER>::mk], s))
           : (void)0), ...);
     return s;
 }
 
-template <class R, bool TO_CUM, int I>
+template <class R, bool TO_CUM, int ORDER, int I>
 __device__ __forceinline__ void cum_one(R* m, R* c, R m0, R im0) {
-    const R s = cum_sum<R, I>(c, m, std::make_integer_sequence<int, 27>{});
+    constexpr int order = I % 3 + I / 3 % 3 + I / 9;
+    if constexpr (TO_CUM && order > ORDER) return;   // a cumulant nothing reads
+    const R s = cum_sum<R, ORDER, I>(c, m, std::make_integer_sequence<int, 27>{});
     if constexpr (TO_CUM && !std::is_same<R, double>::value && (I == 1 || I == 3 || I == 9)) {
         // the velocity J/rho in float, corrected to the rounded quotient:
         // J (1/rho) rounds 1/rho once more, and with rho near 1 from below
@@ -1619,21 +1624,21 @@ __device__ __forceinline__ void cum_one(R* m, R* c, R m0, R im0) {
     } else if (TO_CUM) {
         c[I] = (m[I] - s) * im0;
     } else {
-        m[I] = fma(c[I], m0, s);
+        m[I] = order > ORDER ? s : fma(c[I], m0, s);
     }
 }
 
 // one reciprocal of m0 instead of 26 divisions (the float path is
 // arithmetic-bound here)
-template <class R, bool TO_CUM, int... I>
+template <class R, bool TO_CUM, int ORDER, int... I>
 __device__ __forceinline__ void cum_convert_seq(R* m, R* c, std::integer_sequence<int, I...>) {
     const R m0 = m[0], im0 = R(1) / m0;
-    (cum_one<R, TO_CUM, I + 1>(m, c, m0, im0), ...);  // i = 1..26 in order
+    (cum_one<R, TO_CUM, ORDER, I + 1>(m, c, m0, im0), ...);  // i = 1..26 in order
 }
 
-template <class R, bool TO_CUM>
+template <class R, bool TO_CUM, int ORDER>
 __device__ __forceinline__ void cum_convert(R* m, R* c) {
-    cum_convert_seq<R, TO_CUM>(m, c, std::make_integer_sequence<int, 26>{});
+    cum_convert_seq<R, TO_CUM, ORDER>(m, c, std::make_integer_sequence<int, 26>{});
 }
 
 // Run() = RunBoundaries() then CollisionMRT (Dynamics.c.Rt:226-290,
@@ -1721,42 +1726,19 @@ __device__ __forceinline__ void cum_ib(R* f, unsigned nt, const uint16_t* cut, s
     }
 }
 
-// SMAG: the d3q27_cumulant_SMAG build (par[7] = Smag).  AVG: the AVG
-// builds; av (null: no averages kept) points at the node's first averaged
-// density, the k-th at av[k*NN], in the order avgP, varUX, varUY, varUZ,
-// varUXUY, varUXUZ, varUYUZ, avgdxu2, avgdyv2, avgdzw2, avgUX, avgUY,
-// avgUZ.  On collision nodes they gain dxu^2, dyv^2, dzw^2 of the collision
-// (Dynamics.c.Rt:410-414) and P, u, u_i u_j of the post-collision
-// populations (getP, getU_: 0 on Wall nodes; Dynamics.c.Rt:507-518).
-template <class R, bool GLOB, bool SMAG = false, bool AVG = false>
-__device__ __forceinline__ void cum_node(R* f, unsigned nt, const double* par, const double* zr, double* g,
-                                         double* av = nullptr, size_t NN = 0) {
-    cum_boundaries<R, GLOB>(f, nt, zr, g);
-    if ((nt & 0x80u) == 0) return;  // MRT
+// The collision in cumulants of the moments m (Dynamics.c.Rt:329-422), w0 the
+// relaxation of the second order.  ORDER: the highest cumulant that is not
+// zero afterwards, 3, or 2 where Omega is 1 (its default): the third order is
+// then relaxed to zero, so it is neither formed nor carried back.  That gives
+// the same values (what the third order left was products with zero added to
+// sums) with fewer operations in both transforms: the f16s step of
+// 160x128x96 is bound by its instructions and went from 58.6 to 57 us.
+template <class R, bool SMAG, bool AVG, int ORDER>
+__device__ __forceinline__ void cum_relax(R* m, R* c, R w0, unsigned nt, const double* par, double* av, size_t NN) {
     const R Fx = (R)par[3], Fy = (R)par[4], Fz = (R)par[5];
-    R m[27], c[27];
-#pragma unroll
-    for (int i = 0; i < 27; i++) m[i] = f[i];
-    cum_fwd(m);
-    const R rho = m[0];
-    if (GLOB) {
-        // getU_: 0 on Wall nodes, else (J + F/2)/rho
-        const bool wall = ((nt >> 3) & 0xFu) == 10u;
-        const R ux = wall ? R(0) : (m[1] + Fx / R(2)) / rho;
-        const R uy = wall ? R(0) : (m[3] + Fy / R(2)) / rho;
-        const R uz = wall ? R(0) : (m[9] + Fz / R(2)) / rho;
-        g[0] += (double)rho; g[9] += zr[3];
-        g[1] += (double)ux; g[9] += zr[4];
-        g[5] += (double)rho; g[9] += zr[8];
-        g[6] += (double)(rho * ux); g[9] += zr[9];
-        g[7] += (double)(rho * uy); g[9] += zr[10];
-        g[8] += (double)(rho * uz); g[9] += zr[11];
-    }
-    R w0 = ((nt >> 3) & 0xFu) != 0 ? R(1) / (R(3) * (R)par[1] + R(0.5))
-                                    : R(1) / (R(3) * (R)par[0] + R(0.5));
-    const R w1 = R(1);
+    const R rho = m[0], w1 = R(1);
     c[0] = R(1);
-    cum_convert<R, true>(m, c);
+    cum_convert<R, true, ORDER>(m, c);
     if constexpr (SMAG) {
         // Smagorinsky (Dynamics.c.Rt:362-374): tau_t from the deviation of the
         // second cumulants from 1/3; buffer-layer nodes keep nubuffer
@@ -1799,14 +1781,50 @@ __device__ __forceinline__ void cum_node(R* f, unsigned nt, const double* par, c
     c[4] *= R(1) - w0;
     c[12] *= R(1) - w0;
     c[10] *= R(1) - w0;
-    const R om3 = R(1) - (R)par[6];
+    if constexpr (ORDER >= 3) {
+        const R om3 = R(1) - (R)par[6];
 #pragma unroll
-    for (int i = 0; i < 27; i++) {
-        const int o = i % 3 + i / 3 % 3 + i / 9;
-        if (o == 3) c[i] *= om3;
-        if (o > 3) c[i] = R(0);
+        for (int i = 0; i < 27; i++)
+            if (i % 3 + i / 3 % 3 + i / 9 == 3) c[i] *= om3;
     }
-    cum_convert<R, false>(m, c);
+    cum_convert<R, false, ORDER>(m, c);
+}
+
+// SMAG: the d3q27_cumulant_SMAG build (par[7] = Smag).  AVG: the AVG
+// builds; av (null: no averages kept) points at the node's first averaged
+// density, the k-th at av[k*NN], in the order avgP, varUX, varUY, varUZ,
+// varUXUY, varUXUZ, varUYUZ, avgdxu2, avgdyv2, avgdzw2, avgUX, avgUY,
+// avgUZ.  On collision nodes they gain dxu^2, dyv^2, dzw^2 of the collision
+// (Dynamics.c.Rt:410-414) and P, u, u_i u_j of the post-collision
+// populations (getP, getU_: 0 on Wall nodes; Dynamics.c.Rt:507-518).
+template <class R, bool GLOB, bool SMAG = false, bool AVG = false>
+__device__ __forceinline__ void cum_node(R* f, unsigned nt, const double* par, const double* zr, double* g,
+                                         double* av = nullptr, size_t NN = 0) {
+    cum_boundaries<R, GLOB>(f, nt, zr, g);
+    if ((nt & 0x80u) == 0) return;  // MRT
+    const R Fx = (R)par[3], Fy = (R)par[4], Fz = (R)par[5];
+    R m[27], c[27];
+#pragma unroll
+    for (int i = 0; i < 27; i++) m[i] = f[i];
+    cum_fwd(m);
+    const R rho = m[0];
+    if (GLOB) {
+        // getU_: 0 on Wall nodes, else (J + F/2)/rho
+        const bool wall = ((nt >> 3) & 0xFu) == 10u;
+        const R ux = wall ? R(0) : (m[1] + Fx / R(2)) / rho;
+        const R uy = wall ? R(0) : (m[3] + Fy / R(2)) / rho;
+        const R uz = wall ? R(0) : (m[9] + Fz / R(2)) / rho;
+        g[0] += (double)rho; g[9] += zr[3];
+        g[1] += (double)ux; g[9] += zr[4];
+        g[5] += (double)rho; g[9] += zr[8];
+        g[6] += (double)(rho * ux); g[9] += zr[9];
+        g[7] += (double)(rho * uy); g[9] += zr[10];
+        g[8] += (double)(rho * uz); g[9] += zr[11];
+    }
+    R w0 = ((nt >> 3) & 0xFu) != 0 ? R(1) / (R(3) * (R)par[1] + R(0.5))
+                                    : R(1) / (R(3) * (R)par[0] + R(0.5));
+    if (par[6] == 1.0) cum_relax<R, SMAG, AVG, 2>(m, c, w0, nt, par, av, NN);
+    else cum_relax<R, SMAG, AVG, 3>(m, c, w0, nt, par, av, NN);
     cum_inv(m);
 #pragma unroll
     for (int i = 0; i < 27; i++) f[i] = m[i];

@@ -1,0 +1,45 @@
+"""The cumulant collision without its third order (Omega = 1, the default)
+and with it, through the C ABI, on random NodeTypes and boundary conditions."""
+import numpy as np
+import pytest
+
+from conftest import oracle_for_case
+from test_gpu_parity import random_case, rel_max, say
+
+pytestmark = pytest.mark.gpu
+
+
+def with_omega(model, omega, steps=6):
+    case = random_case(model, 11, 8, 5, seed=47, steps=steps)
+    case.settings = [s for s in case.settings if s[0] != "Omega"] + [("Omega", omega)]
+    return case
+
+
+@pytest.mark.parametrize("model", ["d3q27_cumulant", "d3q27_cumulant_SMAG", "d3q27_cumulant_AVG_IB_SMAG"])
+@pytest.mark.parametrize("omega", [1.0, 1.25])
+def test_third_order_f64(oracle_mod, model, omega):
+    """FP64 against the oracle, to the 1e-12 that its other cases are held to."""
+    say(f"third order {model} Omega {omega}")
+    case = with_omega(model, omega)
+    lat, orc = case.build("f64"), oracle_for_case(oracle_mod, case, "f64")
+    for n in (1, 6):
+        lat.iterate(n)
+        orc.iterate(n)
+        assert rel_max(lat.get_f(), orc.get_f()) <= 1e-12, n
+
+
+@pytest.mark.parametrize("model,storage", [("d3q27_cumulant", "f32"), ("d3q27_cumulant", "f16s"),
+                                           ("d3q27_cumulant_SMAG", "f32s"), ("d3q27_cumulant_IB", "bf16s"),
+                                           ("d3q27_cumulant_AVG", "f32s")])
+def test_left_out_third_order_is_exact(model, storage):
+    """Omega = 1 + 2^-40 is 1 in the float collision but not to the test for
+    1, so its third order is formed and multiplied by zero: the values must
+    be those of Omega = 1, where it is left out."""
+    say(f"third order left out {model} {storage}")
+    out = []
+    for omega in (1.0, 1.0 + 2.0 ** -40):
+        lat = with_omega(model, omega).build(storage)
+        lat.iterate(7)
+        out.append((lat.get_f(), lat.globals))
+    assert np.array_equal(out[0][0], out[1][0])
+    assert np.array_equal(out[0][1], out[1][1])
