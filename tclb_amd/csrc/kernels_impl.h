@@ -2021,7 +2021,14 @@ __device__ __forceinline__ void node_update(const StepArgs& a, int row, int xc, 
     // of every address is a 32-bit byte offset (a plane is at most 4 GiB:
     // check_lattice_size refuses larger ones)
     const char* fin = (const char*)a.fin;
-    const size_t pbytes = (size_t)a.pitch * sizeof(T);
+    size_t pbytes = (size_t)a.pitch * sizeof(T);
+    // opaque, and walked from plane to plane by scalar additions: the
+    // optimiser otherwise forms every plane's offset before the loop over the
+    // tile's rows, more scalars than there are, and parks them in the lanes of
+    // vector registers (27 directions: 122 of the 134 vector instructions of
+    // the entry, 63 to read them back, and a 64-bit vector addition per store;
+    // the f16s cumulant step of 160x128x96 57 us so, 51 this way)
+    asm volatile("" : "+s"(fin), "+s"(pbytes));
     // d3q19 and the 2D models in a shifted format collide on the stored
     // deviations f - w
     constexpr bool DEV = (is_d3q19<MODEL> || L::Q == 9) && S::shifted;
@@ -2033,6 +2040,7 @@ __device__ __forceinline__ void node_update(const StepArgs& a, int row, int xc, 
         // loop, serializing the pulls).  Not for the 27-velocity models,
         // whose capped steps would then spill.
         T v[Q];
+        const char* plane = fin;
 #pragma unroll
         for (int i = 0; i < Q; i++) {
             // source node x - e_i with periodic wrap
@@ -2040,7 +2048,9 @@ __device__ __forceinline__ void node_update(const StepArgs& a, int row, int xc, 
             const int sy = L::ey(i) > 0 ? ym : (L::ey(i) < 0 ? yp : y);
             const int sz = L::ez(i) > 0 ? zm : (L::ez(i) < 0 ? zp : z);
             const unsigned src = (unsigned)sx + (unsigned)nx * ((unsigned)sy + (unsigned)ny * (unsigned)sz);
-            v[i] = *(gptr<const T>)(fin + (size_t)i * pbytes + src * (unsigned)sizeof(T));
+            v[i] = *(gptr<const T>)(plane + src * (unsigned)sizeof(T));
+            plane += pbytes;
+            asm volatile("" : "+s"(plane));
         }
         if constexpr (Q < 27) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -2089,23 +2099,27 @@ __device__ __forceinline__ void node_update(const StepArgs& a, int row, int xc, 
             d2q9_node<R, MODEL == MODEL_D2Q9_SRT_DRAG, GLOB>(f, nt, (R)a.par[0], (R)a.par[1], zr, g);
         }
         // streaming stores: nothing reads them back this step
-        char* fout = (char*)a.fout;
-        if constexpr (S::stochastic) {
-            // direction 2j rounds with word j, 2j + 1 with word j << 16
-            uint32_t w = sr_word0(n, a.sr_key);
+        char* plane = (char*)a.fout;
+        unsigned at = n * (unsigned)sizeof(T);
+        asm volatile("" : "+s"(plane), "+v"(at));
+        // stochastic rounding: direction 2j rounds with word j, 2j + 1 with
+        // word j << 16
+        uint32_t w = 0;
+        if constexpr (S::stochastic) w = sr_word0(n, a.sr_key);
 #pragma unroll
-            for (int i = 0; i < Q; i++) {
+        for (int i = 0; i < Q; i++) {
+            T out;
+            if constexpr (S::stochastic) {
                 const uint32_t r = (i & 1) ? w << 16 : w;
-                __builtin_nontemporal_store(DEV ? S::unraw_sr(f[i], r) : S::put_sr(f[i], (R)L::w(i), r),
-                                            (gptr<T>)(fout + (size_t)i * pbytes + n * (unsigned)sizeof(T)));
+                out = DEV ? S::unraw_sr(f[i], r) : S::put_sr(f[i], (R)L::w(i), r);
                 if (i & 1) w = xorshift32(w);
+            } else {
+                out = DEV ? S::unraw(f[i]) : S::put(f[i], (R)L::w(i));
             }
-            return;
+            __builtin_nontemporal_store(out, (gptr<T>)(plane + at));
+            plane += pbytes;
+            asm volatile("" : "+s"(plane));
         }
-#pragma unroll
-        for (int i = 0; i < Q; i++)
-            __builtin_nontemporal_store(DEV ? S::unraw(f[i]) : S::put(f[i], (R)L::w(i)),
-                                        (gptr<T>)(fout + (size_t)i * pbytes + n * (unsigned)sizeof(T)));
     }
 }
 

@@ -111,13 +111,15 @@ __global__ void __launch_bounds__(TX * TY) k_march3d(StepArgs a, int tiles_x, in
     // the pulls of layer z: a scalar base and one of the 32-bit offsets each
     const auto fetch = [&](int z) {
         const int zm = z == 0 ? nz - 1 : z - 1, zp = z == nz - 1 ? 0 : z + 1;
-        const char* base = (const char*)a.fin;
+        const char* plane = (const char*)a.fin;
+        asm volatile("" : "+s"(plane));
+        const size_t at[3] = {(size_t)zm * layer * sizeof(T), (size_t)z * layer * sizeof(T), (size_t)zp * layer * sizeof(T)};
         nt_next = *(gptr<const uint16_t>)((const char*)(a.flags + (size_t)z * layer) + off[1][1] / (unsigned)(sizeof(T) / 2));
 #pragma unroll
         for (int i = 0; i < Q; i++) {
-            const int sz = L::ez(i) > 0 ? zm : (L::ez(i) < 0 ? zp : z);
-            v[i] = *(gptr<const T>)(base + (size_t)i * pbytes + (size_t)sz * layer * sizeof(T) +
-                                    off[1 - L::ey(i)][1 - L::ex(i)]);
+            v[i] = *(gptr<const T>)(plane + at[1 - L::ez(i)] + off[1 - L::ey(i)][1 - L::ex(i)]);
+            plane += pbytes;
+            asm volatile("" : "+s"(plane));
         }
     };
     unsigned nt0 = 0, nt1 = 0, nt2 = 0;  // NodeTypes of layers z, z - 1 and z - 2
@@ -155,8 +157,13 @@ __global__ void __launch_bounds__(TX * TY) k_march3d(StepArgs a, int tiles_x, in
                 uint32_t w = 0;
                 if constexpr (S::stochastic)
                     w = sr_word0((unsigned)x + (unsigned)nx * (unsigned)y + layer * (unsigned)z2, sr_key(a.sr_step + 1u, a.sr_seed));
-                char* base = (char*)a.fout + (size_t)z2 * layer * sizeof(T);
-                store_node<S, L, DEV>(f, w, [&](int i, T out) { *(gptr<T>)(base + (size_t)i * pbytes + off[1][1]) = out; });
+                char* plane = (char*)a.fout + (size_t)z2 * layer * sizeof(T);
+                asm volatile("" : "+s"(plane));
+                store_node<S, L, DEV>(f, w, [&](int, T out) {
+                    *(gptr<T>)(plane + off[1][1]) = out;
+                    plane += pbytes;
+                    asm volatile("" : "+s"(plane));
+                });
             }
         }
         if (it < layers + 2) {
