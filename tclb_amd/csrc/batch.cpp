@@ -520,14 +520,15 @@ void Batch::GetQuantity(int id, int q, double* out, double scale) {
     upload_zones();
     StepArgs a = case_args(c);
     if ((phase_ ^ c.parity) & 1) a.fin = arena_.base() + c.snap_off[1];
-    const size_t bytes = c.N * (model->quantities[q].vector ? 3 : 1) * sizeof(double);
-    double* d = nullptr;
-    hip_check(hipMalloc((void**)&d, bytes), "hipMalloc(quantity)");
-    hipError_t e = launch_quantity(model->id, storage, q, a, 0, 0, 0, c.nx, c.ny, c.nz, scale, d, stream_);
-    if (e == hipSuccess) e = hipMemcpyAsync(out, d, bytes, hipMemcpyDeviceToHost, stream_);
-    if (e == hipSuccess) e = hipStreamSynchronize(stream_);
-    (void)hipFree(d);
-    hip_check(e, "GetQuantity");
+    const size_t row = (size_t)c.nx * (model->quantities[q].vector ? 3 : 1) * sizeof(double);
+    if (c.nz == 1)
+        readback_.read(c.ny, row, out, stream_, [&](size_t y, size_t n, double* dst) {
+            return launch_quantity(model->id, storage, q, a, 0, (int)y, 0, c.nx, (int)n, 1, scale, dst, stream_);
+        });
+    else
+        readback_.read(c.nz, row * c.ny, out, stream_, [&](size_t z, size_t n, double* dst) {
+            return launch_quantity(model->id, storage, q, a, 0, 0, (int)z, c.nx, c.ny, (int)n, scale, dst, stream_);
+        });
 }
 
 void Batch::GetDensity(int id, int q, double* out) {

@@ -163,6 +163,7 @@ private:
     int tb_k_ = 0;
     bool tune_auto_ = true;  // no tuning was set or timed
     BlockedBatch blocked_;
+    Readback readback_;
     std::vector<int> order_;  // case id of device slot i
     hipStream_t stream_ = nullptr;
     hipEvent_t ev0_ = nullptr, ev1_ = nullptr;

@@ -111,6 +111,8 @@ Lattice::Lattice(const ModelDef* m, int nx_, int ny_, int nz_, int storage_)
     flat_ = flat_pays(nx);
     const int G = kernel_nglobals(m->id);
     hip_check(hipMalloc((void**)&d_glob_, MAX_GLOBALS * sizeof(double)), "hipMalloc(globals)");
+    hip_check(hipHostMalloc((void**)&h_glob_, MAX_GLOBALS * sizeof(double), hipHostMallocDefault),
+              "hipHostMalloc(globals)");
     hip_check(hipMemsetAsync(d_glob_, 0, MAX_GLOBALS * sizeof(double), stream_), "hipMemset(globals)");
     globals_.assign(G, 0.0);
     // the class of a node: its NodeType bits below the zone; the bulk class
@@ -141,6 +143,7 @@ Lattice::~Lattice() {
     if (d_zone_) (void)hipFree(d_zone_);
     if (d_gpart_) (void)hipFree(d_gpart_);
     if (d_glob_) (void)hipFree(d_glob_);
+    if (h_glob_) (void)hipHostFree(h_glob_);
     if (d_list_) (void)hipFree(d_list_);
     if (ev0_) (void)hipEventDestroy(ev0_);
     if (ev1_) (void)hipEventDestroy(ev1_);
@@ -669,18 +672,17 @@ void Lattice::Iterate(int niter, int iter_type) {
         snap_ = 1 - snap_;
     }
     hip_check(hipEventRecord(ev1_, stream_), "event record");
+    const bool read_globals = last_glob || (iter_type & ITER_INTEG);
+    if (read_globals) fetch_globals();
     hip_check(hipStreamSynchronize(stream_), "Iterate");
     float ms = 0;
     hip_check(hipEventElapsedTime(&ms, ev0_, ev1_), "event elapsed");
     last_ms_ = ms;
     kernel_ms_ += ms;
     iter_ += niter;
-    if (last_glob) {
-        std::fill(globals_.begin(), globals_.end(), 0.0);
-        calcGlobals();
-    } else if (iter_type & ITER_INTEG) {
-        calcGlobals();
-    }
+    if (last_glob) std::fill(globals_.begin(), globals_.end(), 0.0);
+    if (read_globals)
+        for (size_t i = 0; i < globals_.size(); i++) globals_[i] += h_glob_[i];
 }
 
 void Lattice::clearGlobals() { std::fill(globals_.begin(), globals_.end(), 0.0); }
@@ -689,29 +691,40 @@ void Lattice::clearGlobals() { std::fill(globals_.begin(), globals_.end(), 0.0);
 // (The non-zonal InObj objective term there is empty for these models:
 // every InObj weight is zonal and already added on the device.)
 void Lattice::calcGlobals() {
-    std::vector<double> tab(globals_.size());
-    hip_check(hipMemcpyAsync(tab.data(), d_glob_, tab.size() * sizeof(double), hipMemcpyDeviceToHost, stream_),
+    fetch_globals();
+    hip_check(hipStreamSynchronize(stream_), "calcGlobals");
+    for (size_t i = 0; i < globals_.size(); i++) globals_[i] += h_glob_[i];
+}
+
+// the device values on their way to h_glob_ (the stream's next
+// synchronisation completes them), the device cleared
+void Lattice::fetch_globals() {
+    hip_check(hipMemcpyAsync(h_glob_, d_glob_, MAX_GLOBALS * sizeof(double), hipMemcpyDeviceToHost, stream_),
               "read globals");
     hip_check(hipMemsetAsync(d_glob_, 0, MAX_GLOBALS * sizeof(double), stream_), "clear globals");
-    hip_check(hipStreamSynchronize(stream_), "calcGlobals");
-    for (size_t i = 0; i < tab.size(); i++) globals_[i] += tab[i];
 }
 
 void Lattice::GetQuantity(int q, const Region& over, double* out, double scale) {
     if (q < 0 || q >= (int)model->quantities.size()) throw std::out_of_range("quantity id");
     if (!region_in(over, nx, ny, nz)) throw std::out_of_range("quantity region outside the lattice");
-    const size_t n = (size_t)over.nx * over.ny * over.nz;
-    if (n == 0) return;
-    const size_t count = n * (model->quantities[q].vector ? 3 : 1);
-    double* d_out = nullptr;
-    hip_check(hipMalloc((void**)&d_out, count * sizeof(double)), "hipMalloc(quantity)");
-    try {
-        GetQuantityStaged(q, over, out, scale, d_out, count);
-    } catch (...) {
-        (void)hipFree(d_out);
-        throw;
+    if ((size_t)over.nx * over.ny * over.nz == 0) return;
+    upload_zone();
+    const StepArgs a = args(snap_, 1 - snap_, false);
+    const size_t row = over.nx * (model->quantities[q].vector ? 3 : 1) * sizeof(double);
+    // the region in chunks of layers, or of the rows of one layer where that
+    // is all there is or a layer is too large for a chunk
+    if (over.nz > 1 && row * over.ny <= Readback::CHUNK) {
+        readback_.read(over.nz, row * over.ny, out, stream_, [&](size_t z, size_t n, double* dst) {
+            return launch_quantity(model->id, storage, q, a, over.dx, over.dy, over.dz + (int)z, over.nx, over.ny,
+                                   (int)n, scale, dst, stream_);
+        });
+        return;
     }
-    hip_check(hipFree(d_out), "hipFree(quantity)");
+    for (int z = 0; z < over.nz; z++)
+        readback_.read(over.ny, row, (char*)out + row * over.ny * z, stream_, [&](size_t y, size_t n, double* dst) {
+            return launch_quantity(model->id, storage, q, a, over.dx, over.dy + (int)y, over.dz + z, over.nx, (int)n,
+                                   1, scale, dst, stream_);
+        });
 }
 
 void Lattice::GetQuantityStaged(int q, const Region& over, double* out, double scale, double* staging,

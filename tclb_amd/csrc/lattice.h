@@ -10,6 +10,7 @@
 
 #include "kernels.h"
 #include "model.h"
+#include "readback.h"
 
 namespace tclbx {
 
@@ -131,6 +132,7 @@ private:
     int blocked_k() const { return tb_k_ > 1 && !(sorted_ && model->dim == 3) ? tb_k_ : 1; }
     int graph_len() const;
     void drop_graph();
+    void fetch_globals();
     void tune_rows();
     void run_graph_steps(int nsteps);
     void ensure_list();
@@ -148,6 +150,7 @@ private:
     double* d_zone_ = nullptr;
     double* d_gpart_ = nullptr;
     double* d_glob_ = nullptr;
+    double* h_glob_ = nullptr;  // pinned: what fetch_globals read
     std::vector<double> globals_;
     int nblocks_ = 0, block_ = 256, bpr_ = 1, rpb_ = 1;
     bool flat_ = false;  // plain steps walk runs of the linear index
@@ -174,6 +177,7 @@ private:
     int tb_k_ = 0;
     bool tb_auto_ = false;
     Blocking tb_split3d_;
+    Readback readback_;
     std::vector<Blocking> tb_split_;  // the split of k steps per launch, by k, as needed
 };
 
