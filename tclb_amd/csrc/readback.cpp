@@ -80,35 +80,31 @@ private:
 }  // namespace
 
 Readback::~Readback() {
-    for (int b = 0; b < 2; b++) {
-        if (dev_[b]) (void)hipFree(dev_[b]);
-        if (pinned_[b]) (void)hipHostFree(pinned_[b]);
-        if (done_[b]) (void)hipEventDestroy(done_[b]);
-    }
+    if (dev_) (void)hipFree(dev_);
+    if (pinned_) (void)hipHostFree(pinned_);
+    for (hipEvent_t e : done_)
+        if (e) (void)hipEventDestroy(e);
 }
 
 // buffers of at least `bytes`: powers of two up to CHUNK, so that a region
-// that grows from read to read does not allocate on each
+// that grows from read to read does not allocate on each.  Both buffers of a
+// kind are one allocation: the first read of a lattice pays for it.
 void Readback::reserve(size_t bytes, bool device) {
     size_t want = 4096;
     while (want < bytes && want < CHUNK) want *= 2;
     want = std::max(want, bytes);
     if (pinned_cap_ < bytes) {
         pinned_cap_ = 0;
-        for (char*& p : pinned_) {
-            if (p) (void)hipHostFree(p);
-            p = nullptr;
-        }
-        for (char*& p : pinned_) hip_check(hipHostMalloc((void**)&p, want, hipHostMallocDefault), "hipHostMalloc(field staging)");
+        if (pinned_) (void)hipHostFree(pinned_);
+        pinned_ = nullptr;
+        hip_check(hipHostMalloc((void**)&pinned_, 2 * want, hipHostMallocDefault), "hipHostMalloc(field staging)");
         pinned_cap_ = want;
     }
     if (device && dev_cap_ < bytes) {
         dev_cap_ = 0;
-        for (char*& p : dev_) {
-            if (p) (void)hipFree(p);
-            p = nullptr;
-        }
-        for (char*& p : dev_) hip_check(hipMalloc((void**)&p, want), "hipMalloc(field staging)");
+        if (dev_) (void)hipFree(dev_);
+        dev_ = nullptr;
+        hip_check(hipMalloc((void**)&dev_, 2 * want), "hipMalloc(field staging)");
         dev_cap_ = want;
     }
 }
@@ -120,14 +116,13 @@ void Readback::read(size_t units, size_t unit_bytes, void* out, hipStream_t stre
     std::lock_guard<std::mutex> one(m_);
     if (total <= DIRECT) {
         reserve(total, false);
-        hip_check(eval(0, units, (double*)pinned_[0]), "field kernel");
+        hip_check(eval(0, units, (double*)pinned_), "field kernel");
         hip_check(hipStreamSynchronize(stream), "read field");
-        std::memcpy(out, pinned_[0], total);
+        std::memcpy(out, pinned_, total);
         return;
     }
-    // at least four chunks where a chunk of an eighth of a CHUNK still is
-    // worth its launch and copy, so that small fields overlap too
-    const size_t chunk = std::max(unit_bytes, std::min(CHUNK, std::max(CHUNK / 8, total / 4)));
+    // four chunks, of 1 MB at least, so that small fields overlap too
+    const size_t chunk = std::max(unit_bytes, std::min(CHUNK, std::max(CHUNK / 16, total / 4)));
     const size_t per = std::min(units, chunk / unit_bytes), chunks = (units + per - 1) / per;
     reserve(per * unit_bytes, true);
     for (hipEvent_t& e : done_)
@@ -136,12 +131,12 @@ void Readback::read(size_t units, size_t unit_bytes, void* out, hipStream_t stre
         hipStream_t s;
         ~Drain() { (void)hipStreamSynchronize(s); }
     } drain{stream};
-    // a thread for every 2 MB (for every 512 kB: U of 1024x256 400 us, not 324)
+    // a thread for every 2 MB (for every 512 kB: U of 1024x256 400 us, not 311)
     Copier copier((unsigned)std::min<size_t>(8, 1 + total / (size_t(2) << 20)));
     const auto start = [&](size_t c) {
         const size_t b = c & 1, first = c * per, n = std::min(per, units - first);
-        hip_check(eval(first, n, (double*)dev_[b]), "field kernel");
-        hip_check(hipMemcpyAsync(pinned_[b], dev_[b], n * unit_bytes, hipMemcpyDeviceToHost, stream), "read field");
+        hip_check(eval(first, n, (double*)(dev_ + b * dev_cap_)), "field kernel");
+        hip_check(hipMemcpyAsync(pinned_ + b * pinned_cap_, dev_ + b * dev_cap_, n * unit_bytes, hipMemcpyDeviceToHost, stream), "read field");
         hip_check(hipEventRecord(done_[b], stream), "event record");
     };
     start(0);
@@ -149,7 +144,7 @@ void Readback::read(size_t units, size_t unit_bytes, void* out, hipStream_t stre
         if (c + 1 < chunks) start(c + 1);
         const size_t b = c & 1, first = c * per, n = std::min(per, units - first);
         hip_check(hipEventSynchronize(done_[b]), "read field");
-        copier.copy((char*)out + first * unit_bytes, pinned_[b], n * unit_bytes);
+        copier.copy((char*)out + first * unit_bytes, pinned_ + b * pinned_cap_, n * unit_bytes);
     }
 }
 

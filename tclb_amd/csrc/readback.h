@@ -21,7 +21,7 @@ namespace tclbx {
 // caller's pages, which several threads share; a small one by calls.  Against
 // a device allocation per read and a copy to pageable memory (U of d3q19 256^3,
 // 403 MB, 38.0 -> 9.6 ms; of 256x128x128 9.7 -> 2.9; of 128x96x64, 19 MB,
-// 1.09 -> 0.67; of d2q9 1024x256, 6 MB, 403 -> 324 us; of 128x32 70 -> 22 us).
+// 1.09 -> 0.67; of d2q9 1024x256, 6 MB, 403 -> 311 us; of 128x32 70 -> 22 us).
 class Readback {
 public:
     Readback() = default;
@@ -40,8 +40,8 @@ public:
 private:
     void reserve(size_t bytes, bool device);
     std::mutex m_;
-    char* dev_[2] = {nullptr, nullptr};
-    char* pinned_[2] = {nullptr, nullptr};
+    char* dev_ = nullptr;     // two buffers of dev_cap_ bytes, one after the other
+    char* pinned_ = nullptr;  // two of pinned_cap_ bytes
     hipEvent_t done_[2] = {nullptr, nullptr};
     size_t dev_cap_ = 0, pinned_cap_ = 0;
 };
