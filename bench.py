@@ -32,13 +32,13 @@ def log(msg):
 
 
 def traffic_table():
-    """HBM bytes per launch measured by rocprofv3 --pmc (FETCH_SIZE,
+    """HBM bytes per time step measured by rocprofv3 --pmc (FETCH_SIZE,
     WRITE_SIZE), scaled by the copy-kernel calibration; see profiles/."""
     p = os.path.join(ROOT, "profiles", "traffic_d3q19_porous256.json")
     if not os.path.exists(p):
         return {}
     with open(p) as f:
-        return json.load(f).get("per_launch_bytes", {})
+        return json.load(f).get("per_step_bytes", {})
 
 
 def _oracle_mlups(n, seconds, threads):
@@ -250,7 +250,9 @@ def main():
         lat.iterate(args.steps, tclb_amd.ITER_NORM | tclb_amd.ITER_LASTGLOB)
         wall = time.perf_counter() - t0
         ev_ms, _ = lat.timing()
-        bpn = lat.bytes_per_node()
+        # the least bytes of a step: a launch of k steps moves the state once
+        k = max(1, lat.temporal_blocking)
+        bpn = lat.bytes_per_node() / k
         per_launch_ms = ev_ms / args.steps
         achieved = bpn * N / (per_launch_ms * 1e-3) / 1e9
         g = lat.global_dict()
@@ -262,6 +264,7 @@ def main():
             "ms_per_step": wall * 1e3 / args.steps,
             "kernel_ms": per_launch_ms,
             "bytes_per_node": bpn,
+            "steps_per_launch": k,
             "achieved_GBs": achieved,
             "roofline_frac": achieved / HBM_PEAK_GBS,
             "steps_run": args.warmup + args.steps,
