@@ -607,11 +607,19 @@ void Lattice::tune_rows() {
     drop_graph();
 }
 
+// Blocked steps have no rows per tile.  A step of the AVG builds adds to the
+// averages, so these run no trial steps; one row per tile is their fastest
+// (us per step with 1, 2 and 4: d3q27_cumulant_AVG 160x128x96 f64 261, 287,
+// 287, f16s 146, 150, 161; 128x128x64 f32 87, 88, 90).
+bool Lattice::times_rows() const {
+    return tune_rpt_ && blocked_k() == 1 && N >= (1u << 20) && model->averages.empty();
+}
+
 void Lattice::Prepare() {
     upload_zone();
     ensure_list();
     choose_blocking();
-    if (tune_rpt_ && blocked_k() == 1 && N >= (1u << 20)) tune_rows();
+    if (times_rows()) tune_rows();
     if (graph_steps_ >= 2 && !sr_) {
         run_graph_steps(0);  // capture only
         hip_check(hipStreamSynchronize(stream_), "Prepare");
@@ -630,8 +638,8 @@ void Lattice::Iterate(int niter, int iter_type) {
     const int k = every_glob ? 1 : blocked_k();
     // lattices large enough for the tiling to matter are tuned once, on
     // the first Iterate that runs enough steps to repay the trial launches
-    // (or earlier, by Prepare); blocked steps have no rows per tile
-    if (tune_rpt_ && k == 1 && niter >= 16 && N >= (1u << 20)) tune_rows();
+    // (or earlier, by Prepare)
+    if (niter >= 16 && times_rows()) tune_rows();
     hip_check(hipEventRecord(ev0_, stream_), "event record");
     int i = 0;
     // leading plain steps until snapshot 0 is current, then whole graph

@@ -134,6 +134,7 @@ private:
     void drop_graph();
     void fetch_globals();
     void tune_rows();
+    bool times_rows() const;
     void run_graph_steps(int nsteps);
     void ensure_list();
 

@@ -3,6 +3,8 @@ and with it, through the C ABI, on random NodeTypes and boundary conditions."""
 import numpy as np
 import pytest
 
+import tclb_amd
+
 from conftest import oracle_for_case
 from test_gpu_parity import random_case, rel_max, say
 
@@ -43,3 +45,27 @@ def test_left_out_third_order_is_exact(model, storage):
         out.append((lat.get_f(), lat.globals))
     assert np.array_equal(out[0][0], out[1][0])
     assert np.array_equal(out[0][1], out[1][1])
+
+
+def test_timing_of_the_tiles_leaves_the_averages():
+    """The averages of a lattice large enough to have its tiles timed
+    (2^20 nodes) are those of one whose tiles are given: trial steps, which
+    run on the current snapshot, would add to them."""
+    nx, ny, nz = 128, 128, 64
+    rng = np.random.default_rng(8)
+    flags = np.where(rng.random((nz, ny, nx)) < 0.05, 0, tclb_amd.Model("d3q27_cumulant_AVG").flag("MRT"))
+    runs = []
+    for rows in (0, 1):
+        lat = tclb_amd.Lattice("d3q27_cumulant_AVG", nx, ny, nz, "f16s")
+        lat.set_flags(flags.astype(np.uint16))
+        lat.set_setting("ForceX", 1e-5)
+        lat.rows_per_tile = rows
+        lat.init()
+        if rows == 0:
+            lat.prepare()
+        lat.iterate(20)
+        runs.append(lat.get_averages())
+        lat.close()
+    assert np.abs(runs[0]["avgP"]).max() > 0 or np.abs(runs[0]["avgUX"]).max() > 0
+    for k, v in runs[0].items():
+        assert np.array_equal(v, runs[1][k]), k
