@@ -233,8 +233,14 @@ StepArgs Batch::case_args(const Case& c) const {
     a.pitch = (long long)c.pitch;
     a.nx = c.nx; a.ny = c.ny; a.nz = c.nz;
     // flat runs for every step (a tuning that asks for them), or by default
-    // for the plain steps of the cases whose rows leave lanes idle
-    a.flat = tune_.flat ? 3 : (tune_auto_ && flat_pays(c.nx) ? 1 : 0);
+    // for the plain steps of the cases whose rows leave lanes idle.  Rows of
+    // half a block keep row segments in the 4- and 8-byte formats: whole
+    // waves of such a block idle and take nothing from a step that HBM
+    // bounds (four d3q19 boxes, us per step on row segments against runs:
+    // 128x128x128 f64 507 / 521, f32s 261 / 276; 128x200x200 f64 1161 / 1166;
+    // d3q27 f32 128x128x127 388 / 424; six 128^3 f16s 228 / 196).
+    const bool half = 2 * c.nx == tune_.block && storage_bytes(storage) >= 4;
+    a.flat = tune_.flat ? 3 : (tune_auto_ && flat_pays(c.nx) && !half ? 1 : 0);
     a.inv_nx = 1.0 / c.nx;
     a.inv_ny = 1.0 / c.ny;
     a.bpr = (c.nx + tune_.block - 1) / tune_.block;

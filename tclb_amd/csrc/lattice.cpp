@@ -37,8 +37,14 @@ int pick_block(int nx) {
 // a small lattice's blocks are all full.  us per step, best row segments
 // against runs of 256: d3q19 f64 157x131x97 151 / 114, 96^3 54.8 / 53.8, f16s
 // 71x150x100 29.8 / 17.8, 160x159x155 66.9 / 55.5; d3q27 f32 129x97x113 98.3 /
-// 68.3; d3q27_cumulant f16s 160x128x96 65.8 / 53.7; at 256^3 the two are equal
-// (f16s 235.7 / 235.1).
+// 68.3; at 256^3 the two are equal (f16s 235.7 / 235.1).  Where row segments
+// leave no lane idle either (nx a multiple of the block), runs still win on
+// small lattices, which hold more full blocks of them (f16s 64^3 6.7 / 4.9,
+// 128x96x64 14.8 / 14.3, 192x64x48 13.1 / 11.7, 640x64x48 30.7 / 28.7; f64
+// 46.8-48.1 / 46.8 and 118 / 119 for the last two), and large ones go either
+// way with the planes' strides (f16s 128x400x320 250 / 238, 384x512x512 1517 /
+// 1544, 640^3 4000 / 4095; d3q27 f32 384x512x512 4100 / 4000): tune_rows
+// times both there.
 bool flat_pays(int nx) { return nx % 256 != 0; }
 
 int default_graph_steps() {
@@ -108,7 +114,7 @@ Lattice::Lattice(const ModelDef* m, int nx_, int ny_, int nz_, int storage_)
     }
     hip_check(hipMalloc((void**)&d_zone_, std::max<size_t>(1, zone_.size()) * sizeof(double)), "hipMalloc(zone)");
     set_block(pick_block(nx));
-    flat_ = flat_pays(nx);
+    flat_ = may_flat_ = flat_pays(nx);
     const int G = kernel_nglobals(m->id);
     hip_check(hipMalloc((void**)&d_glob_, MAX_GLOBALS * sizeof(double)), "hipMalloc(globals)");
     hip_check(hipHostMalloc((void**)&h_glob_, MAX_GLOBALS * sizeof(double), hipHostMallocDefault),
@@ -153,7 +159,7 @@ Lattice::~Lattice() {
 void Lattice::set_block(int b) {
     if (b != 64 && b != 128 && b != 256) throw std::invalid_argument("block must be 64, 128 or 256");
     block_ = b;
-    flat_ = false;   // a block that the caller sets is a row segment's
+    flat_ = may_flat_ = false;   // a block that the caller sets is a row segment's
     bpr_ = (nx + b - 1) / b;
     nblocks_ = bpr_ * ny * nz;
     rpb_ = globals_rows_per_block((long long)ny * nz, bpr_);
@@ -581,29 +587,42 @@ void Lattice::set_rows_per_tile(int r) {
     drop_graph();
 }
 
-// Times plain steps with 1, 2 and 4 rows per tile and keeps the fastest.
-// Every trial step reads the current snapshot and writes the other one,
-// which the next real step overwrites: the state does not change.  Which
-// is fastest depends on the model, the storage format and the occupancy
+// Times plain steps with 1, 2 and 4 rows per tile, on runs of the linear
+// index and, where these leave no lane idle, on row segments, and keeps the
+// fastest.  Every trial step reads the current snapshot and writes the other
+// one, which the next real step overwrites: the state does not change.
+// Which is fastest depends on the model, the storage format, the occupancy
 // the kernel reaches (one row for FP64 d3q19, more for the 16-bit formats
-// of heavier node types).
+// of heavier node types) and on how the planes' strides fall on the memory
+// channels.
 void Lattice::tune_rows() {
     tune_rpt_ = false;
+    const char* log = std::getenv("TCLBX_TUNE_LOG");
     float best = 0;
     int best_r = rpt_;
-    for (int r : {1, 2, 4}) {
-        if (r > 1 && (long long)ny * nz < 4LL * r) continue;
-        rpt_ = r;
-        launch(snap_, 1 - snap_, false);  // warm-up
-        hip_check(hipEventRecord(ev0_, stream_), "event record");
-        for (int k = 0; k < 3; k++) launch(snap_, 1 - snap_, false);
-        hip_check(hipEventRecord(ev1_, stream_), "event record");
-        hip_check(hipStreamSynchronize(stream_), "tune rows");
-        float ms = 0;
-        hip_check(hipEventElapsedTime(&ms, ev0_, ev1_), "event elapsed");
-        if (best == 0 || ms < best) { best = ms; best_r = r; }
+    bool best_flat = flat_;
+    for (bool flat : {true, false}) {
+        if (flat ? !may_flat_ : may_flat_ && nx % block_ != 0) continue;
+        for (int r : {1, 2, 4}) {
+            if (r > 1 && (long long)ny * nz < 4LL * r) continue;
+            rpt_ = r;
+            flat_ = flat;
+            launch(snap_, 1 - snap_, false);  // warm-up
+            hip_check(hipEventRecord(ev0_, stream_), "event record");
+            for (int k = 0; k < 3; k++) launch(snap_, 1 - snap_, false);
+            hip_check(hipEventRecord(ev1_, stream_), "event record");
+            hip_check(hipStreamSynchronize(stream_), "tune rows");
+            float ms = 0;
+            hip_check(hipEventElapsedTime(&ms, ev0_, ev1_), "event elapsed");
+            if (log && std::atoi(log) != 0)
+                std::fprintf(stderr, "tclbx: %s %dx%dx%d %s: %d rows per tile on %s: %.1f us per step\n",
+                             model->name.c_str(), nx, ny, nz, storage_name(storage), r,
+                             flat ? "runs" : "row segments", 1e3 * ms / 3);
+            if (best == 0 || ms < best) { best = ms; best_r = r; best_flat = flat; }
+        }
     }
     rpt_ = best_r;
+    flat_ = best_flat;
     drop_graph();
 }
 

@@ -154,7 +154,8 @@ private:
     double* h_glob_ = nullptr;  // pinned: what fetch_globals read
     std::vector<double> globals_;
     int nblocks_ = 0, block_ = 256, bpr_ = 1, rpb_ = 1;
-    bool flat_ = false;  // plain steps walk runs of the linear index
+    // plain steps walk runs of the linear index; they may (no block was set)
+    bool flat_ = false, may_flat_ = false;
     int plain_block() const { return flat_ ? 256 : block_; }
     hipStream_t stream_ = nullptr;
     hipEvent_t ev0_ = nullptr, ev1_ = nullptr;

@@ -121,3 +121,23 @@ def test_marching_tiles_are_bit_identical(model, storage, shape):
         v[0:5 * v[1::5].size:5] = v[1::5]
         a.set_flags(flags)
         b.set_flags(flags)
+
+
+def test_single_steps_are_timed_on_runs_and_on_row_segments(capfd, monkeypatch):
+    """A lattice whose row segments leave no lane idle times both forms of its
+    tiles; one whose rows end inside a block keeps runs, and one that was given
+    a block keeps row segments."""
+    monkeypatch.setenv("TCLBX_TUNE_LOG", "1")
+    for nx, block, forms in ((128, None, {"runs", "row segments"}), (136, None, {"runs"}),
+                             (128, 64, {"row segments"}), (256, None, {"row segments"})):
+        say(f"forms timed at {nx}, block {block}")
+        lat = tclb_amd.Lattice("d3q19", nx, 128, 8192 // nx + 1, "f16s")
+        lat.set_flags(np.full((lat.nz, lat.ny, lat.nx), lat.spec.flag("MRT"), np.uint16))
+        if block:
+            lat.set_block(block)
+        lat.init()
+        capfd.readouterr()
+        lat.prepare()
+        log = [line for line in capfd.readouterr().err.splitlines() if "rows per tile on" in line]
+        assert {line.split(" on ")[1].split(":")[0] for line in log} == forms, log
+        lat.close()
