@@ -191,13 +191,16 @@ int tclbx_get_timing(const tclbx_lattice* h, double* last_ms, double* total_ms);
 /* Algorithmic HBM bytes per node and step: 2*Q*sizeof(storage) + 2 (flag),
  * the reference's GB/s formula with the storage width (src/main.cpp:127). */
 int tclbx_bytes_per_node(const tclbx_lattice* h, double* bytes);
-/* Launch shape: threads per block along x (64, 128 or 256); 0 = default. */
+/* Launch shape of the single steps: threads per block along x (64, 128 or 256);
+ * 0 = default.  A 3D lattice given one (or a number of rows below) takes single
+ * steps (tclbx_set_temporal_blocking). */
 int tclbx_set_block(tclbx_lattice* h, int block);
 /* Steps per captured hipGraph replay in tclbx_iterate (0 = no graph). */
 int tclbx_set_graph_steps(tclbx_lattice* h, int steps);
 /* Rows walked by one block of a plain step: 1, 2 or 4; 0 (the default) times
  * the three on the first long tclbx_iterate of a lattice of 2^20 nodes or
- * more and keeps the fastest (the state is not changed).  A launch-shape
+ * more that takes single steps and keeps no averages, and keeps the fastest
+ * (the state is not changed).  A launch-shape
  * choice of this engine; the reference's shape is fixed (32x4 threads). */
 int tclbx_set_rows_per_tile(tclbx_lattice* h, int rows);
 int tclbx_get_rows_per_tile(const tclbx_lattice* h, int* rows);
@@ -240,8 +243,9 @@ int tclbx_set_stochastic_rounding(tclbx_lattice* h, int on, unsigned seed);
  * steps, bit for bit, stochastic rounding included.  Steps with Globals take
  * the single step.  Batches of these models step the same way.  Lattices of
  * the 3D models take two steps per launch, bit for bit those of single steps,
- * where their model, storage format and size make that faster; 0 or 1 turns
- * that off too (-1 and larger numbers are refused).  The environment's
+ * where their model, storage format and size make that faster, unless they
+ * have the sorted dispatch or were given a block or rows per tile; 0 or 1
+ * turns that off too (-1 and larger numbers are refused).  The environment's
  * TCLBX_TEMPORAL_BLOCKING=k (k >= 0; 2 and more for the 2D models only)
  * fixes it for new lattices and batches.  No counterpart in the reference, which launches
  * one kernel per iteration (src/Lattice.cu.Rt:1246-1297). */

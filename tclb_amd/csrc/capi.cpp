@@ -360,16 +360,7 @@ int tclbx_bytes_per_node(const tclbx_lattice* h, double* bytes) {
 int tclbx_set_block(tclbx_lattice* h, int block) {
     CHECK_H(h);
     return guard([&]() {
-        int b = block;
-        if (b == 0) {
-            b = 256;
-            long long best = -1;
-            for (int c : {256, 128, 64}) {
-                long long w = (long long)((h->lat->nx + c - 1) / c) * c - h->lat->nx;
-                if (best < 0 || w < best) { best = w; b = c; }
-            }
-        }
-        h->lat->set_block(b);
+        h->lat->set_block(block);
         return TCLBX_OK;
     });
 }

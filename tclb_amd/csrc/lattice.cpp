@@ -113,8 +113,7 @@ Lattice::Lattice(const ModelDef* m, int nx_, int ny_, int nz_, int storage_)
         hip_check(hipMemsetAsync(d_extra_, 0, ab, stream_), "hipMemset(extra densities)");
     }
     hip_check(hipMalloc((void**)&d_zone_, std::max<size_t>(1, zone_.size()) * sizeof(double)), "hipMalloc(zone)");
-    set_block(pick_block(nx));
-    flat_ = may_flat_ = flat_pays(nx);
+    set_block(0);
     const int G = kernel_nglobals(m->id);
     hip_check(hipMalloc((void**)&d_glob_, MAX_GLOBALS * sizeof(double)), "hipMalloc(globals)");
     hip_check(hipHostMalloc((void**)&h_glob_, MAX_GLOBALS * sizeof(double), hipHostMallocDefault),
@@ -157,9 +156,13 @@ Lattice::~Lattice() {
 }
 
 void Lattice::set_block(int b) {
-    if (b != 64 && b != 128 && b != 256) throw std::invalid_argument("block must be 64, 128 or 256");
+    if (b != 0 && b != 64 && b != 128 && b != 256) throw std::invalid_argument("block must be 0, 64, 128 or 256");
+    block_set_ = b != 0;
+    if (b == 0) b = pick_block(nx);
     block_ = b;
-    flat_ = may_flat_ = false;   // a block that the caller sets is a row segment's
+    // a block that the caller sets is a row segment's
+    flat_ = may_flat_ = !block_set_ && flat_pays(nx);
+    if (!block_set_ && !rows_set_) tune_rpt_ = true;   // the default shape is timed anew
     bpr_ = (nx + b - 1) / b;
     nblocks_ = bpr_ * ny * nz;
     rpb_ = globals_rows_per_block((long long)ny * nz, bpr_);
@@ -582,8 +585,10 @@ void Lattice::resetAverage() {
 
 void Lattice::set_rows_per_tile(int r) {
     if (r != 0 && r != 1 && r != 2 && r != 4) throw std::invalid_argument("rows per tile must be 0, 1, 2 or 4");
+    rows_set_ = r != 0;
     tune_rpt_ = r == 0;
     rpt_ = r == 0 ? 1 : r;
+    if (r == 0) flat_ = may_flat_;
     drop_graph();
 }
 

@@ -112,7 +112,7 @@ public:
     // single step.  3D lattices take two steps per launch where that is
     // faster (blocking3d); 0 turns that off too, other numbers are refused.
     void set_temporal_blocking(int k);
-    int temporal_blocking() const { return tb_k_; }
+    int temporal_blocking() const { return tb_k_ > 1 && blocked_k() == 1 ? 0 : tb_k_; }
 
     const ModelDef* model;
     const int nx, ny, nz, storage;
@@ -127,9 +127,11 @@ private:
     const Blocking& blocking(int k);
     void set_blocking(StepArgs& a, int k);
     void choose_blocking();
-    // steps per blocked launch; the sorted dispatch of a 3D lattice, which its
-    // caller asked for, keeps single steps
-    int blocked_k() const { return tb_k_ > 1 && !(sorted_ && model->dim == 3) ? tb_k_ : 1; }
+    // steps per blocked launch; a 3D lattice whose caller asked for the sorted
+    // dispatch or for a tile shape keeps the single steps that have them
+    int blocked_k() const {
+        return tb_k_ > 1 && !(model->dim == 3 && (sorted_ || block_set_ || rows_set_)) ? tb_k_ : 1;
+    }
     int graph_len() const;
     void drop_graph();
     void fetch_globals();
@@ -156,6 +158,7 @@ private:
     int nblocks_ = 0, block_ = 256, bpr_ = 1, rpb_ = 1;
     // plain steps walk runs of the linear index; they may (no block was set)
     bool flat_ = false, may_flat_ = false;
+    bool block_set_ = false, rows_set_ = false;  // by the caller
     int plain_block() const { return flat_ ? 256 : block_; }
     hipStream_t stream_ = nullptr;
     hipEvent_t ev0_ = nullptr, ev1_ = nullptr;

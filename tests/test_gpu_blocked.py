@@ -141,3 +141,27 @@ def test_single_steps_are_timed_on_runs_and_on_row_segments(capfd, monkeypatch):
         log = [line for line in capfd.readouterr().err.splitlines() if "rows per tile on" in line]
         assert {line.split(" on ")[1].split(":")[0] for line in log} == forms, log
         lat.close()
+
+
+def test_a_set_tile_shape_takes_single_steps():
+    """A block or a number of rows per tile that the caller sets is what a 3D
+    lattice steps in; 0 gives the choice back, and so does sorted dispatch
+    when it is turned off.  The getter says what is in use."""
+    say("a set tile shape on a marching lattice")
+    case = random_case("d3q19", 159, 130, 75, seed=5)
+    a = case.build("f64")
+    a.iterate(3)
+    assert a.temporal_blocking == 2
+    for on, off in ((lambda: a.set_block(64), lambda: a.set_block(0)),
+                    (lambda: setattr(a, "rows_per_tile", 2), lambda: setattr(a, "rows_per_tile", 0)),
+                    (lambda: setattr(a, "sorted_dispatch", True), lambda: setattr(a, "sorted_dispatch", False))):
+        on()
+        a.iterate(3)
+        assert a.temporal_blocking == 0
+        off()
+        a.iterate(3)
+        assert a.temporal_blocking == 2
+    b = case.build("f64")
+    b.temporal_blocking = 0
+    b.iterate(3 * 7)
+    assert same(a.get_f(), b.get_f())
