@@ -238,8 +238,8 @@ int tclbx_set_stochastic_rounding(tclbx_lattice* h, int on, unsigned seed);
  * (2-15) time steps per launch, on tiles held in LDS or, up to 5 steps on
  * larger lattices, by waves that march through the lattice with the steps
  * in between in registers; 0 or 1 turns it off; -1, the default of these
- * models, takes the steps per launch that the lattice's size and storage
- * format call for when it first iterates.  Results are those of single
+ * models, takes the steps per launch (one, too) that the lattice's size and
+ * storage format call for when it first iterates.  Results are those of single
  * steps, bit for bit, stochastic rounding included.  Steps with Globals take
  * the single step.  Batches of these models step the same way.  Lattices of
  * the 3D models take two steps per launch, bit for bit those of single steps,

@@ -93,9 +93,10 @@ struct Blocking {
 };
 // the models the blocked steps cover
 bool blocked2d_model(int model);
-// The split for a lattice of nx x ny nodes: of k steps per launch, or with k =
-// 0 of the best number of steps (kernels.hip says why the lines lie there).
-Blocking blocking2d(int nx, int ny, int storage, int k);
+// The split for a lattice of nx x ny nodes (sr: with stochastic rounding): of k
+// steps per launch, or with k = 0 of the best number of steps, which may be
+// one (kernels.hip says how it is found).
+Blocking blocking2d(int model, int nx, int ny, int storage, bool sr, int k);
 // two steps per launch of a 3D lattice: marching tiles (tx x ty columns, rows =
 // layers along z), or k = 1 where single steps are as fast
 Blocking blocking3d(int model, int nx, int ny, int nz, int storage);

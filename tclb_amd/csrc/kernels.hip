@@ -120,28 +120,52 @@ double weight(int model, int q) {
 }
 }  // namespace
 
-// Lines measured on d2q9_SRT in f64 and f32s and on d2q9_drag in f16s (us per
-// step, tiles against marching waves at each one's best split):
-//   f64   1501x333 8.8 / 10.6, 2048x512 17.8 / 15.6, 2048x1024 31.5 / 27.7,
-//         4096x2048 122 / 95
-//   f32s  2048x1024 13.3 / 14.3, 4096x2048 52.4 / 43.6
-//   f16s  2048x1024 14.4 / 15.3, 4096x2048 54.6 / 44.6
-// The waves need 3,000 or more of them to cover each other's latencies, each
-// with enough rows to pay for the 2(k-1) it steps beside them; the FP64 tile
-// holds one or two blocks per CU, the float tiles twice as many.
-static bool blocking2d_marches(long long nodes, int storage) {
-    return nodes >= (storage == ST_F64 ? 1ll << 20 : 1ll << 22);
+// What a 2D lattice takes: single steps, marching waves or LDS tiles, whichever
+// has the least estimated time per step.  The coefficients (us; MB of
+// populations moved) are fitted to the times of 46 lattices, from 64x64 to
+// 4096x2048 and among them 4x262144, 57x20000 and 1000000x4, with single steps,
+// waves of k = 3 to 5 and tiles of k = 3 to 5 and 256 to 1024 nodes: within 6
+// to 15% (rms) of each, and the steps they choose take 2% longer than the best
+// of all on average (lines by size alone: 17%, up to 4.2 times).  us per step
+// of single steps, waves and tiles where sizes alone mislead: f32s 256x256 3.6,
+// 4.7 and, with k = 3 and 5, 2.5 and 1.8; 1500x1000 21.6, 8.1, 13.4; f16s
+// 4x262144, where a strip or tile wastes most of its columns, 10, 56, 18; f64
+// 8x131072 33, 66, 18; with stochastic rounding, whose random streams a blocked
+// step draws in its halo too, f16s 2000x1500 22, 24, 22 (without 22, 16, 19).
+// (k = 4 tiles are left out: the better of 3 and 5 is at most 10% behind.)
+struct StepCost2d {
+    double single, single_mb;                            // a step
+    double tile, tile_mb, tile_rounds;                   // a launch of tiles, a round of blocks,
+    double tile_stage, tile_wave, tile_block;            // a round's step, of a SIMD's waves, of a block's
+    double march, march_mb, march_hbm, march_row, march_wave;   // waves: a row's step, of a SIMD's waves
+};
+static const StepCost2d& step_cost2d(int model, int storage, bool sr) {
+    static const StepCost2d costs[2][4] = {
+        // d2q9_SRT(_drag): f64, f32 and f32s, 16 bit, 16 bit with stochastic rounding
+        {{2.91, 0.181, 3.61, 0.127, 0, 0.85, 0.13, 0, 6.48, 0.0434, 0.0468, 0.317, 0.177},
+         {2.56, 0.186, 4.12, 0.227, 0, 0.0942, 0.035, 0.0932, 6.02, 0.0784, 0.0549, 0.196, 0.0326},
+         {2.64, 0.220, 3.70, 0.313, 0, 0.150, 0.070, 0.107, 6.94, 0.0424, 0.0471, 0.196, 0.0856},
+         {3.09, 0.218, 4.23, 0.242, 0, 0.170, 0.130, 0, 8.21, 0.0348, 0.0612, 0.226, 0.185}},
+        // d2q9(_drag), the same
+        {{3.09, 0.182, 1.91, 0.133, 0, 0.897, 0.156, 0.203, 7.54, 0.0261, 0.0499, 0.372, 0.244},
+         {2.79, 0.187, 3.65, 0.207, 0, 0.262, 0.0509, 0.128, 6.98, 0.0375, 0.0495, 0.282, 0.0891},
+         {2.73, 0.192, 3.40, 0.284, 0, 0.217, 0.090, 0.116, 6.85, 0.0395, 0.0418, 0.196, 0.106},
+         {3.21, 0.191, 4.22, 0.222, 0, 0.196, 0.159, 0, 7.28, 0.0511, 0.020, 0.247, 0.220}}};
+    const int f = storage == ST_F64 ? 0 : storage == ST_F32 || storage == ST_F32S ? 1 : sr ? 3 : 2;
+    return costs[model == MODEL_D2Q9 || model == MODEL_D2Q9_DRAG][f];
 }
+static double mb2d(double nodes, int storage) { return nodes * 9 * storage_bytes(storage) / 1e6; }
 
 static int strips2d(int nx, int k) { return (nx + 64 - 2 * (k - 1) - 1) / (64 - 2 * (k - 1)); }
 
-// Marching waves for n lattices of `nodes` nodes in all.
-// f64 4096x2048: k 3 104, 4 98, 5 95 us per step; 2048x1024: k 3 30.6, 4 27.7,
-// 5 30.5.  f32s 4096x2048: 60, 50, 44.  f16s: 44.6, 46.7, 50.5 (its
-// conversions make a step dearer than the bytes it saves).  Rows for about
-// 3,000 waves, between what pays for the extra rows and what evens out the
-// last round (f64 8-12 to 24, float 8 to 12 measured).
-static BlockedBatch march_split(const int2* sizes, int n, long long nodes, int storage, int k, Blocking* cases) {
+// Marching waves for n lattices of `nodes` nodes in all, and their us per
+// step.  With k = 0 the number of steps by size: f64 4096x2048 k 3 104, 4 98, 5
+// 95 us per step; 2048x1024 k 3 30.6, 4 27.7, 5 30.5; f32s 4096x2048 60, 50, 44;
+// f16s 44.6, 46.7, 50.5 (its conversions make a step dearer than the bytes it
+// saves).  Rows for about 3,000 waves, between what pays for the extra rows
+// and what evens out the last round (f64 8-12 to 24, float 8 to 12 measured).
+static BlockedBatch march_split(const StepCost2d& c, const int2* sizes, int n, long long nodes, int storage, int k,
+                                Blocking* cases, double& us) {
     const bool f64 = storage == ST_F64, half = storage == ST_F16S || storage == ST_BF16S;
     BlockedBatch b;
     b.k = k ? k : f64 ? (nodes >= 1ll << 22 ? 5 : 4) : half ? 3 : 5;
@@ -149,25 +173,32 @@ static BlockedBatch march_split(const int2* sizes, int n, long long nodes, int s
     for (int i = 0; i < n; i++) rows += (long long)strips2d(sizes[i].x, b.k) * sizes[i].y;
     b.rows = (int)std::min<long long>(f64 ? 24 : 12, std::max<long long>(f64 ? 6 : 8, (rows + 3071) / 3072));
     b.threads = 256;
+    double wave_rows = 0;   // rows that the waves walk, and the longest walk
+    int longest = 0;
     for (int i = 0; i < n; i++) {
         cases[i] = Blocking();
         cases[i].k = b.k;
         cases[i].rows = std::min(b.rows, sizes[i].y);
+        const int walk = cases[i].rows + 2 * (b.k - 1);
+        wave_rows += (double)strips2d(sizes[i].x, b.k) * ((sizes[i].y + cases[i].rows - 1) / cases[i].rows) * walk;
+        longest = std::max(longest, walk);
     }
+    const double mb = mb2d(64 * wave_rows + (double)nodes, storage);
+    const bool hbm = mb2d(2.0 * (double)nodes, storage) > 200;   // past the Infinity Cache
+    us = (c.march + (c.march_mb + (hbm ? c.march_hbm : 0)) * mb) / b.k + c.march_row * longest +
+         c.march_wave * wave_rows / 1024;
     return b;
 }
 
-// The tiles of the least estimated time per step.  A launch takes rounds x (A
-// + k x stage), stage = s0 + s1 x waves per SIMD, fitted to single rounds of
-// 128x32 and 1024x128 (f64: 16x16 tiles, one wave per SIMD, 0.84 us a stage,
-// 32x16 1.33, 32x32 2.25; f32s 0.55, 1.06, 1.37; f16s 0.83, -, 2.1) and to
-// the rounds of 1501x333 (f64 32x16, two rounds of 12.5 us at k = 3).
-static BlockedBatch tile_split(const int2* sizes, int n, int storage, const std::vector<int>& ks, Blocking* cases) {
-    const double A = 2.8, s0 = 0.4, s1 = storage == ST_F64 ? 0.47 : storage == ST_F32 || storage == ST_F32S ? 0.22 : 0.26;
+// The tiles of the least estimated time per step, among ks steps per launch:
+// a round of blocks takes k stages, in each of which a SIMD steps its waves
+// one after the other.
+static BlockedBatch tile_split(const StepCost2d& c, const int2* sizes, int n, long long nodes, int storage,
+                               const std::vector<int>& ks, Blocking* cases, double& us) {
     const int capacity = storage == ST_F64 ? 6 : 8;   // waves per SIMD
     std::vector<Blocking> trial(n);
     BlockedBatch best;
-    double best_t = 1e300;
+    us = 1e300;
     for (int k : ks)
         for (int threads : {256, 512, 1024}) {
             long long tiles = 0;
@@ -192,9 +223,11 @@ static BlockedBatch tile_split(const int2* sizes, int n, int storage, const std:
             const long long per_cu = (tiles + 255) / 256;
             double rounds = (double)tiles / (256.0 * fit);
             rounds = rounds < 4 ? std::ceil(rounds) : rounds + 0.5;
-            const double t = rounds * (A + k * (s0 + s1 * waves * std::min<long long>(fit, per_cu))) / k;
-            if (t < best_t) {
-                best_t = t;
+            const double t = (c.tile + c.tile_mb * mb2d((double)tiles * threads + (double)nodes, storage) +
+                              c.tile_rounds * rounds) / k + c.tile_block * waves +
+                             rounds * (c.tile_stage + c.tile_wave * waves * std::min<long long>(fit, per_cu));
+            if (t < us) {
+                us = t;
                 best.k = k; best.rows = 0; best.threads = threads;
                 for (int i = 0; i < n; i++) {
                     cases[i] = trial[i];
@@ -205,21 +238,35 @@ static BlockedBatch tile_split(const int2* sizes, int n, int storage, const std:
     return best;
 }
 
-Blocking blocking2d(int nx, int ny, int storage, int k) {
+Blocking blocking2d(int model, int nx, int ny, int storage, bool sr, int k) {
+    const StepCost2d& c = step_cost2d(model, storage, sr);
     const int2 size = make_int2(nx, ny);
-    Blocking b;
-    if (k <= MARCH2D_MAX_K && blocking2d_marches((long long)nx * ny, storage))
-        march_split(&size, 1, (long long)nx * ny, storage, k, &b);
-    else
-        tile_split(&size, 1, storage, k ? std::vector<int>{k} : std::vector<int>{3, 5}, &b);
-    return b;
+    const long long nodes = (long long)nx * ny;
+    Blocking tile, march;
+    double tile_us, march_us = 1e300;
+    tile_split(c, &size, 1, nodes, storage, k ? std::vector<int>{k} : std::vector<int>{3, 5}, &tile, tile_us);
+    if (k <= MARCH2D_MAX_K) march_split(c, &size, 1, nodes, storage, k, &march, march_us);
+    const double single_us = c.single + c.single_mb * mb2d(2.0 * (double)nodes, storage);
+    if (k == 0 && single_us < std::min(tile_us, march_us)) return Blocking();
+    return march_us < tile_us ? march : tile;
 }
 
+// A batch marches by whole launches of k steps and takes the rest as single
+// steps, which short calls pay for (Globals every 10 steps), so it marches only
+// where that gains most; its tiles' coefficients are those of single rounds of
+// 128x32 and 1024x128 (f64: 16x16 tiles, one wave per SIMD, 0.84 us a stage,
+// 32x16 1.33, 32x32 2.25; f32s 0.55, 1.06, 1.37; f16s 0.83, -, 2.1).
 BlockedBatch blocking2d_batch(const int2* sizes, int n, int storage, int k, Blocking* cases) {
+    StepCost2d c = {};
+    c.tile_rounds = 2.8;
+    c.tile_stage = 0.4;
+    c.tile_wave = storage == ST_F64 ? 0.47 : storage == ST_F32 || storage == ST_F32S ? 0.22 : 0.26;
     long long nodes = 0;
     for (int i = 0; i < n; i++) nodes += (long long)sizes[i].x * sizes[i].y;
-    if (k <= MARCH2D_MAX_K && blocking2d_marches(nodes, storage)) return march_split(sizes, n, nodes, storage, k, cases);
-    return tile_split(sizes, n, storage, k ? std::vector<int>{k} : std::vector<int>{3, 4, 5}, cases);
+    double us;
+    if (k <= MARCH2D_MAX_K && nodes >= (storage == ST_F64 ? 1ll << 20 : 1ll << 22))
+        return march_split(c, sizes, n, nodes, storage, k, cases, us);
+    return tile_split(c, sizes, n, nodes, storage, k ? std::vector<int>{k} : std::vector<int>{3, 4, 5}, cases, us);
 }
 
 // The march's time is rounds of blocks (one per CU: the tile fills its LDS) x

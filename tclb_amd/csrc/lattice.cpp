@@ -128,11 +128,11 @@ Lattice::Lattice(const ModelDef* m, int nx_, int ny_, int nz_, int storage_)
     bulk_val_ = coll ? coll->value : 0u;
     if (const char* e = std::getenv("TCLBX_SORTED_DISPATCH")) sorted_ = std::atoi(e) != 0 && coll != nullptr;
     // (2D: k steps per launch; 3D: two, by size only)
-    tb_auto_ = true;
+    tb_auto_ = tb_own_ = true;
     if (const char* e = std::getenv("TCLBX_TEMPORAL_BLOCKING"))
         if (std::atoi(e) >= 0 && (blocked2d_model(m->id) || std::atoi(e) < 2)) {
             tb_k_ = std::min(TB_MAX_K, std::atoi(e));
-            tb_auto_ = false;
+            tb_auto_ = tb_own_ = false;
         }
     hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
 }
@@ -329,6 +329,9 @@ void Lattice::set_stochastic_rounding(bool on, unsigned seed) {
     if (on && storage != ST_F16S && storage != ST_BF16S)
         throw std::invalid_argument(std::string("stochastic rounding applies to the 16-bit formats f16s and bf16s, not ") +
                                     storage_name(storage));
+    // the steps per launch of a lattice left to choose depend on it
+    if (sr_ != on && tb_own_) tb_auto_ = true;
+    tb_split_.clear();
     sr_ = on;
     sr_seed_ = seed;
     drop_graph();
@@ -341,14 +344,14 @@ void Lattice::set_temporal_blocking(int k) {
     if ((k > 1 || k == -1) && !blocked2d_model(model->id))
         throw std::invalid_argument("temporal blocking applies to d2q9_SRT, d2q9_SRT_drag, d2q9 and d2q9_drag, not " +
                                     model->name);
-    tb_auto_ = k == -1;
+    tb_auto_ = tb_own_ = k == -1;
     tb_k_ = k == -1 ? 0 : k;
     drop_graph();
 }
 
 const Blocking& Lattice::blocking(int k) {
     if (tb_split_.empty()) tb_split_.resize(TB_MAX_K + 1);
-    if (tb_split_[k].k != k) tb_split_[k] = blocking2d(nx, ny, storage, k);
+    if (tb_split_[k].k != k) tb_split_[k] = blocking2d(model->id, nx, ny, storage, sr_, k);
     return tb_split_[k];
 }
 
@@ -362,13 +365,14 @@ void Lattice::choose_blocking() {
         drop_graph();
         return;
     }
-    const Blocking b = blocking2d(nx, ny, storage, 0);
-    tb_k_ = b.k;
+    const Blocking b = blocking2d(model->id, nx, ny, storage, sr_, 0);
+    tb_k_ = b.k > 1 ? b.k : 0;
     if (const char* e = std::getenv("TCLBX_TUNE_LOG"); e && std::atoi(e) != 0)
         std::fprintf(stderr, "tclbx: %s %dx%d %s: %d steps per launch, %s\n", model->name.c_str(), nx, ny,
                      storage_name(storage), b.k,
-                     b.rows ? ("waves of " + std::to_string(b.rows) + " rows").c_str()
-                            : ("tiles of " + std::to_string(b.tx) + "x" + std::to_string(b.ty)).c_str());
+                     b.k == 1 ? "single steps"
+                     : b.rows ? ("waves of " + std::to_string(b.rows) + " rows").c_str()
+                              : ("tiles of " + std::to_string(b.tx) + "x" + std::to_string(b.ty)).c_str());
     drop_graph();
 }
 

@@ -180,7 +180,8 @@ private:
     bool sr_ = false;
     unsigned sr_seed_ = 0;
     int tb_k_ = 0;
-    bool tb_auto_ = false;
+    // left to choose when it next iterates; the number was or will be its own choice
+    bool tb_auto_ = false, tb_own_ = false;
     Blocking tb_split3d_;
     Readback readback_;
     std::vector<Blocking> tb_split_;  // the split of k steps per launch, by k, as needed

@@ -19,7 +19,8 @@ def same(a, b):
 @pytest.mark.parametrize("model,storage,nx,ny,k", [
     ("d2q9_SRT", "f64", 1031, 1021, 2),         # 1,031 = 16 strips of 62 and 39 columns
     ("d2q9_drag", "f64", 1031, 1021, 4),
-    ("d2q9_SRT_drag", "f64", 57, 18500, 5),     # narrower than a strip of 56: its halo wraps onto itself
+    ("d2q9_SRT_drag", "f64", 57, 18500, 5),
+    ("d2q9_SRT_drag", "f64", 50, 21000, 5),     # narrower than a strip of 56: its halo wraps onto itself
     ("d2q9", "f16s", 2053, 2049, 3),
     ("d2q9_SRT", "f32s", 70001, 61, 5),         # rows that a segment of 12 does not divide
 ])
@@ -165,3 +166,22 @@ def test_a_set_tile_shape_takes_single_steps():
     b.temporal_blocking = 0
     b.iterate(3 * 7)
     assert same(a.get_f(), b.get_f())
+
+
+@pytest.mark.parametrize("model,storage,nx,ny,steps", [
+    ("d2q9_SRT", "f64", 4, 262144, (0,)),          # a strip or a tile wastes most of its columns
+    ("d2q9", "f16s", 4, 2000000, (0,)),
+    ("d2q9_SRT_drag", "f64", 8, 131072, (3, 5)),   # tiles, not waves of 64 columns
+    ("d2q9_SRT", "f32s", 256, 256, (5,)),
+    ("d2q9", "f16s", 1, 1, (0, 3, 5)),
+])
+def test_steps_per_launch_by_size(model, storage, nx, ny, steps):
+    """What a lattice left to itself takes, against single steps' bits."""
+    say(f"steps per launch {model} {storage} {nx}x{ny}")
+    case = random_case(model, nx, ny, 1, seed=3)
+    a, b = case.build(storage), case.build(storage)
+    b.temporal_blocking = 0
+    for x in (a, b):
+        x.iterate(8)
+    assert a.temporal_blocking in steps
+    assert same(a.get_f(), b.get_f()) and same(a.globals, b.globals)
