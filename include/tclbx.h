@@ -283,12 +283,16 @@ int tclbx_batch_get_iteration(const tclbx_batch* b, int id, long long* iter);
 int tclbx_batch_get_quantity(tclbx_batch* b, int id, int q, double* out, double scale);
 int tclbx_batch_get_density(tclbx_batch* b, int id, int q, double* out);
 int tclbx_batch_set_density(tclbx_batch* b, int id, int q, const double* in);
-/* time every tile shape (row segments or flat runs of the node index;
- * threads per block 64/128/256; rows per tile 1/2/4), persistent grid size
- * and tile order on the current cases for `steps` steps each, without
- * changing their state, and keep the fastest */
+/* time every tile shape of the single steps (row segments or flat runs of the
+ * node index; threads per block 64/128/256; rows per tile 1/2/4), persistent
+ * grid size and tile order on the current cases for `steps` steps each, and
+ * the several steps per launch of the 2D models (tclbx_set_temporal_blocking),
+ * without changing their state, and keep the fastest; *us_per_step is its
+ * time */
 int tclbx_batch_autotune(tclbx_batch* b, int steps, int* flat, int* block, int* rows_per_tile, int* grid,
                          double* us_per_step);
+/* a tile shape for every step: plain steps of a 2D batch are then single
+ * steps too, until tclbx_batch_autotune chooses anew */
 int tclbx_batch_set_tuning(tclbx_batch* b, int flat, int block, int rows_per_tile, int grid);
 /* stochastic rounding of every case's stores (f16s, bf16s; TCLBX_ERR for
  * the others), each case keyed by its own node index, iteration and `seed`
@@ -300,7 +304,8 @@ int tclbx_batch_set_stochastic_rounding(tclbx_batch* b, int on, unsigned seed);
 /* the order the step walks the tiles in: 0 the tile list's, 1 XCD-
  * contiguous (the k-th of the eight XCDs takes the k-th contiguous run of
  * tiles, so neighbouring rows are pulled through one L2); the autotuner
- * times both.  set < 0 leaves it; *order gets the current one.  No
+ * times both.  Several steps per launch walk their own tiles in order.  set
+ * < 0 leaves it; *order gets the current one.  No
  * counterpart in the reference (batching is this engine's). */
 int tclbx_batch_tile_order(tclbx_batch* b, int set, int* order);
 int tclbx_batch_get_timing(const tclbx_batch* b, double* last_ms, double* total_ms);
@@ -348,7 +353,8 @@ int tclbx_server_poll(tclbx_server* s, int id, int* state, long long* steps, dou
 int tclbx_server_wait_all(tclbx_server* s, double timeout_s, int* idle);
 int tclbx_server_stats(tclbx_server* s, long long* completed, long long* rejected, long long* node_steps,
                        double* busy_s, int* active, int* queued, double* now_s);
-/* tile shape of the server's batch (flat runs of the node index by default) */
+/* tile shape of the server's batch (flat runs of the node index by default);
+ * as tclbx_batch_set_tuning, a 2D server then takes single steps */
 int tclbx_server_set_tuning(tclbx_server* s, int flat, int block, int rows_per_tile, int grid);
 /* stochastic rounding of the served requests' stores, as
  * tclbx_batch_set_stochastic_rounding; taken up by the worker before its next

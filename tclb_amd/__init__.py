@@ -682,6 +682,9 @@ class Batch:
         return cid
 
     def autotune(self, steps=10):
+        """Times the tile shapes of the single steps, and the several steps per
+        launch of the 2D models, on the current cases and keeps the fastest:
+        its us_per_step and the shape of the steps that are single."""
         fl, b, r, g, us = ctypes.c_int(), ctypes.c_int(), ctypes.c_int(), ctypes.c_int(), ctypes.c_double()
         _check(lib().tclbx_batch_autotune(self._h, int(steps), ctypes.byref(fl), ctypes.byref(b), ctypes.byref(r),
                                           ctypes.byref(g), ctypes.byref(us)))
@@ -689,6 +692,7 @@ class Batch:
                 "order": self.tile_order(), "us_per_step": us.value}
 
     def set_tuning(self, block=256, rows_per_tile=1, grid=0, flat=False, order=0):
+        """A tile shape for every step (those of a 2D batch are then single)."""
         _check(lib().tclbx_batch_set_tuning(self._h, int(bool(flat)), int(block), int(rows_per_tile), int(grid)))
         self.tile_order(order)
 

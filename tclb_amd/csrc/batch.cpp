@@ -2,6 +2,7 @@
 #include "batch.h"
 
 #include <algorithm>
+#include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <limits>
@@ -298,7 +299,7 @@ void Batch::rebuild() {
     std::vector<int> first, count;
     blocked_ = BlockedBatch();
     std::vector<Blocking> split(active_.size());
-    if (tb_k_ != 1 && !active_.empty() && blocked2d_model(model->id)) {
+    if (tb_k_ != 1 && !single_ && !active_.empty() && blocked2d_model(model->id)) {
         std::vector<int2> sizes;
         for (auto& kv : active_) sizes.push_back(make_int2(kv.second.nx, kv.second.ny));
         blocked_ = blocking2d_batch(sizes.data(), (int)sizes.size(), storage, tb_k_, split.data());
@@ -360,6 +361,22 @@ void Batch::rebuild() {
     }
     dirty_ = false;
     version_++;
+}
+
+// the device tables of the current cases, if anything about them changed
+void Batch::refresh() {
+    if (!dirty_) return;
+    rebuild();
+    if (const char* e = std::getenv("TCLBX_TUNE_LOG"); e && std::atoi(e) != 0) {
+        int runs = 0;
+        for (auto& kv : active_) runs += case_args(kv.second).flat & 1;
+        std::fprintf(stderr, "tclbx: batch of %d %s %s cases, %lld nodes: %s\n", ncases_dev_, model->name.c_str(),
+                     storage_name(storage), nodes(),
+                     blocked_.k == 1 ? ("single steps, " + std::to_string(runs) + " cases on runs").c_str()
+                                     : (std::to_string(blocked_.k) + " steps per launch, " +
+                                        (blocked_.rows ? "waves of " + std::to_string(blocked_.rows) + " rows"
+                                                       : "tiles of " + std::to_string(blocked_.threads) + " nodes")).c_str());
+    }
 }
 
 void Batch::launch(int phase, bool glob, int k) {
@@ -446,14 +463,14 @@ void Batch::upload_sr_iterations() {
 }
 
 void Batch::Prepare() {
-    if (dirty_) rebuild();
+    refresh();
     upload_zones();
     if (ncases_dev_ > 0 && graph_steps_ >= 2 && !sr_) capture_graph();
 }
 
 void Batch::Iterate(int niter, int iter_type) {
     if (niter < 0) throw std::invalid_argument("negative iteration count");
-    if (dirty_) rebuild();
+    refresh();
     upload_zones();
     if (ncases_dev_ == 0) return;
     int last_glob = iter_type & ITER_LASTGLOB;
@@ -577,6 +594,11 @@ size_t Batch::bytes_per_node_step() const {
 }
 
 void Batch::SetTuning(const Tuning& t) {
+    SetShape(t);
+    single_ = true;
+}
+
+void Batch::SetShape(const Tuning& t) {
     if (t.block != 64 && t.block != 128 && t.block != 256) throw std::invalid_argument("block must be 64, 128 or 256");
     if (t.rpt < 1 || t.rpt > 64) throw std::invalid_argument("rows per tile must be 1..64");
     if (t.grid < 0) throw std::invalid_argument("grid must be >= 0");
@@ -592,16 +614,31 @@ void Batch::SetTileOrder(int order) {
     dirty_ = true;
 }
 
-// Every candidate runs `steps` plain steps from the current snapshot into the
-// other one (the same phase each time), so the state the next Iterate reads
-// is never touched.
+// Every candidate runs plain steps from the current snapshot into the other
+// one (the same phase each time), so the state the next Iterate reads is never
+// touched: `steps` single steps for a tile shape, as many or a few more for the
+// blocked launches of a 2D batch, which come last.  Steps that reread one
+// snapshot find it in the caches where it fits, single steps more of it than
+// blocked ones (a small lattice's trial takes two thirds of its step's time),
+// so the blocked launches stay unless a shape takes less than two thirds of
+// theirs.
 Tuning Batch::Autotune(int steps) {
     if (steps < 1) throw std::invalid_argument("autotune needs at least one step");
     if (active_.empty()) return tune_;
-    const Tuning saved = tune_;
+    const auto time = [&](int launches, const auto& step) {
+        step();  // warm up
+        hip_check(hipEventRecord(ev0_, stream_), "event record");
+        for (int s = 0; s < launches; s++) step();
+        hip_check(hipEventRecord(ev1_, stream_), "event record");
+        hip_check(hipStreamSynchronize(stream_), "autotune");
+        float ms = 0;
+        hip_check(hipEventElapsedTime(&ms, ev0_, ev1_), "event elapsed");
+        return ms * 1e3 / launches;
+    };
     tune_auto_ = false;
+    single_ = true;
     trials_.clear();
-    Tuning best = saved;
+    Tuning best = tune_;
     best.us_per_step = 1e300;
     for (int flat : {0, 1})
     for (int block : {256, 128, 64})
@@ -617,20 +654,23 @@ Tuning Batch::Autotune(int steps) {
                 tune_ = t;
                 rebuild();
                 upload_zones();
-                launch(phase_, false);  // warm up
-                hip_check(hipEventRecord(ev0_, stream_), "event record");
-                for (int s = 0; s < steps; s++) launch(phase_, false);
-                hip_check(hipEventRecord(ev1_, stream_), "event record");
-                hip_check(hipStreamSynchronize(stream_), "autotune");
-                float ms = 0;
-                hip_check(hipEventElapsedTime(&ms, ev0_, ev1_), "event elapsed");
-                t.us_per_step = ms * 1e3 / steps;
+                t.us_per_step = time(steps, [&] { launch(phase_, false); });
                 trials_.push_back(t);
                 if (t.us_per_step < best.us_per_step) best = t;
             }
     tune_ = best;
+    single_ = false;
+    rebuild();
+    if (const int k = blocked_.k; k > 1) {
+        const double us = time((steps + k - 1) / k, [&] { hip_check(launch_blocked(phase_, k, 0), "blocked batch step"); }) / k;
+        if (const char* e = std::getenv("TCLBX_TUNE_LOG"); e && std::atoi(e) != 0)
+            std::fprintf(stderr, "tclbx: autotune: single steps %.3f us per step, %d per launch %.3f us per step\n",
+                         best.us_per_step, k, us);
+        single_ = best.us_per_step < us * 2 / 3;
+        if (!single_) tune_.us_per_step = us;
+    }
     dirty_ = true;
-    return best;
+    return tune_;
 }
 
 }  // namespace tclbx

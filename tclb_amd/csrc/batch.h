@@ -85,11 +85,14 @@ public:
     void GetDensity(int id, int q, double* out);
     void SetDensity(int id, int q, const double* in);
 
-    // time every tile shape / grid candidate on the current cases (steps
-    // that rewrite only the next snapshot, so the state is untouched) and
-    // keep the fastest
+    // time every tile shape / grid candidate of the single steps on the
+    // current cases, and the blocked steps of a 2D batch (all rewrite only the
+    // next snapshot, so the state is untouched), and keep the fastest
     Tuning Autotune(int steps);
+    // the shape of the single steps, which all steps then are; SetShape sets
+    // it for the steps that are single anyway
     void SetTuning(const Tuning& t);
+    void SetShape(const Tuning& t);
     void SetTileOrder(int order);
     // stochastic rounding of every case's stores (16-bit formats only); a
     // case is keyed by its own node index, iteration and `seed`, as a lone
@@ -126,6 +129,7 @@ private:
     };
     StepArgs case_args(const Case& c) const;
     void rebuild();
+    void refresh();
     void upload_zones();
     // one step; k = its index in the current Iterate (stochastic rounding
     // keys a case's step k by the case's iteration + k)
@@ -162,6 +166,7 @@ private:
     // single steps); blocked_ is what the current set of cases got
     int tb_k_ = 0;
     bool tune_auto_ = true;  // no tuning was set or timed
+    bool single_ = false;    // plain steps are single steps: a tuning was set, or timed faster
     BlockedBatch blocked_;
     Readback readback_;
     std::vector<int> order_;  // case id of device slot i

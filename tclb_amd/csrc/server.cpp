@@ -50,7 +50,7 @@ Server::Server(const ModelDef* m, int storage, size_t hbm_budget, int max_chunk)
     t.flat = 1;
     t.block = 256;
     t.rpt = 4;
-    batch_->SetTuning(t);
+    batch_->SetShape(t);
     worker_ = std::thread([this]() { loop(); });
 }
 

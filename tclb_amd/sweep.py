@@ -9,8 +9,8 @@ error of the drag against that FP64 solve: of the drag averaged over the
 last `window` steps (sampled every `every` steps; shedding cases oscillate,
 so the last-step value also carries the phase of the oscillation) and of
 the last step's drag.  --tuning FLAT,BLOCK,ROWS_PER_TILE,GRID,ORDER runs
-that tile shape instead of the autotuner's pick (for profiled runs, whose
-timing misleads the autotuner).  Prints one JSON object.
+single steps in that tile shape instead of the autotuner's pick (for profiled
+runs, whose timing misleads the autotuner).  Prints one JSON object.
 """
 import argparse
 import json

@@ -292,3 +292,43 @@ def test_full_sweep_batch_case_by_case(oracle_mod):
         a, o = f.get_f(cid), orc.get_f()
         assert np.max(np.abs(a - o)) <= 1e-12 * np.max(np.abs(o)), c.name
         glob_close(f.globals(cid), g[:f.nglobals], 1e-10)
+
+
+def tune_log(capfd):
+    return [line for line in capfd.readouterr().err.splitlines() if "batch of" in line]
+
+
+def test_a_set_tuning_takes_single_steps(capfd, monkeypatch):
+    """A tile shape that the caller sets is the one plain steps run in; a 2D
+    batch without one takes several steps per launch."""
+    say("set tuning takes single steps")
+    monkeypatch.setenv("TCLBX_TUNE_LOG", "1")
+    b = tclb_amd.Batch("d2q9_drag", "f16s", capacity_bytes=32 << 20)
+    for c in mixed_cases("d2q9_drag", 4):
+        b.add(c)
+    b.prepare()
+    assert "steps per launch" in tune_log(capfd)[-1]
+    b.set_tuning(block=64, rows_per_tile=2, grid=17)
+    b.prepare()
+    assert "single steps" in tune_log(capfd)[-1]
+
+
+def test_autotune_times_the_steps_that_run(capfd, monkeypatch):
+    """Autotune times the blocked steps of a 2D batch beside the tile shapes of
+    its single steps and keeps what is fastest: us_per_step is that step's."""
+    say("autotune times what runs")
+    monkeypatch.setenv("TCLBX_TUNE_LOG", "1")
+    b = tclb_amd.Batch("d2q9_drag", "f16s", capacity_bytes=64 << 20)
+    ids = [b.add_case(128 + 16 * i, 64) for i in range(4)]
+    for i in ids:
+        b.set_flags(i, np.full(b.shapes[i], b.spec.flag("MRT"), np.uint16))
+        b.init_case(i)
+    capfd.readouterr()
+    t = b.autotune(steps=15)
+    timed = [line for line in capfd.readouterr().err.splitlines() if "autotune" in line]
+    assert len(timed) == 1, timed
+    single, blocked = (float(timed[0].split(w)[1].split()[0]) for w in ("single steps ", "per launch "))
+    # (a shape has to take less than two thirds of the blocked steps' time)
+    assert abs(t["us_per_step"] - (single if single < blocked * 2 / 3 else blocked)) <= 0.002
+    b.prepare()
+    assert ("steps per launch" in tune_log(capfd)[-1]) == (single >= blocked * 2 / 3)
