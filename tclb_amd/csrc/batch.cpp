@@ -543,15 +543,10 @@ void Batch::GetQuantity(int id, int q, double* out, double scale) {
     upload_zones();
     StepArgs a = case_args(c);
     if ((phase_ ^ c.parity) & 1) a.fin = arena_.base() + c.snap_off[1];
-    const size_t row = (size_t)c.nx * (model->quantities[q].vector ? 3 : 1) * sizeof(double);
-    if (c.nz == 1)
-        readback_.read(c.ny, row, out, stream_, [&](size_t y, size_t n, double* dst) {
-            return launch_quantity(model->id, storage, q, a, 0, (int)y, 0, c.nx, (int)n, 1, scale, dst, stream_);
-        });
-    else
-        readback_.read(c.nz, row * c.ny, out, stream_, [&](size_t z, size_t n, double* dst) {
-            return launch_quantity(model->id, storage, q, a, 0, 0, (int)z, c.nx, c.ny, (int)n, scale, dst, stream_);
-        });
+    readback_.read(c.nx, c.ny, c.nz, (model->quantities[q].vector ? 3 : 1) * sizeof(double), out, stream_,
+                   [&](int x, int y, int z, int nx, int ny, int nz, double* dst) {
+                       return launch_quantity(model->id, storage, q, a, x, y, z, nx, ny, nz, scale, dst, stream_);
+                   });
 }
 
 void Batch::GetDensity(int id, int q, double* out) {

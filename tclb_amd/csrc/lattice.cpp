@@ -746,21 +746,11 @@ void Lattice::GetQuantity(int q, const Region& over, double* out, double scale) 
     if ((size_t)over.nx * over.ny * over.nz == 0) return;
     upload_zone();
     const StepArgs a = args(snap_, 1 - snap_, false);
-    const size_t row = over.nx * (model->quantities[q].vector ? 3 : 1) * sizeof(double);
-    // the region in chunks of layers, or of the rows of one layer where that
-    // is all there is or a layer is too large for a chunk
-    if (over.nz > 1 && row * over.ny <= Readback::CHUNK) {
-        readback_.read(over.nz, row * over.ny, out, stream_, [&](size_t z, size_t n, double* dst) {
-            return launch_quantity(model->id, storage, q, a, over.dx, over.dy, over.dz + (int)z, over.nx, over.ny,
-                                   (int)n, scale, dst, stream_);
-        });
-        return;
-    }
-    for (int z = 0; z < over.nz; z++)
-        readback_.read(over.ny, row, (char*)out + row * over.ny * z, stream_, [&](size_t y, size_t n, double* dst) {
-            return launch_quantity(model->id, storage, q, a, over.dx, over.dy + (int)y, over.dz + z, over.nx, (int)n,
-                                   1, scale, dst, stream_);
-        });
+    readback_.read(over.nx, over.ny, over.nz, (model->quantities[q].vector ? 3 : 1) * sizeof(double), out, stream_,
+                   [&](int x, int y, int z, int nx, int ny, int nz, double* dst) {
+                       return launch_quantity(model->id, storage, q, a, over.dx + x, over.dy + y, over.dz + z, nx, ny,
+                                              nz, scale, dst, stream_);
+                   });
 }
 
 void Lattice::GetQuantityStaged(int q, const Region& over, double* out, double scale, double* staging,

@@ -80,71 +80,80 @@ private:
 }  // namespace
 
 Readback::~Readback() {
-    if (dev_) (void)hipFree(dev_);
     if (pinned_) (void)hipHostFree(pinned_);
     for (hipEvent_t e : done_)
         if (e) (void)hipEventDestroy(e);
 }
 
-// buffers of at least `bytes`: powers of two up to CHUNK, so that a region
-// that grows from read to read does not allocate on each.  Both buffers of a
-// kind are one allocation: the first read of a lattice pays for it.
-void Readback::reserve(size_t bytes, bool device) {
-    size_t want = 4096;
-    while (want < bytes && want < CHUNK) want *= 2;
-    want = std::max(want, bytes);
-    if (pinned_cap_ < bytes) {
-        pinned_cap_ = 0;
-        if (pinned_) (void)hipHostFree(pinned_);
-        pinned_ = nullptr;
-        hip_check(hipHostMalloc((void**)&pinned_, 2 * want, hipHostMallocDefault), "hipHostMalloc(field staging)");
-        pinned_cap_ = want;
+// in layers, in the rows of each layer where one is larger than a chunk, or in
+// the nodes of each row
+void Readback::read(int nx, int ny, int nz, size_t node_bytes, void* out, hipStream_t stream, const Eval& eval) {
+    const size_t row = nx * node_bytes, layer = row * ny;
+    char* const to = (char*)out;
+    if (layer == 0 || nz <= 0) return;
+    std::lock_guard<std::mutex> one(m_);
+    if (nz > 1 && layer <= CHUNK) {
+        read_units(nz, layer, to, stream, [&](int z, int n, double* d) { return eval(0, 0, z, nx, ny, n, d); });
+        return;
     }
-    if (device && dev_cap_ < bytes) {
-        dev_cap_ = 0;
-        if (dev_) (void)hipFree(dev_);
-        dev_ = nullptr;
-        hip_check(hipMalloc((void**)&dev_, 2 * want), "hipMalloc(field staging)");
-        dev_cap_ = want;
+    for (int z = 0; z < nz; z++) {
+        if (row <= CHUNK) {
+            read_units(ny, row, to + layer * z, stream, [&](int y, int n, double* d) { return eval(0, y, z, nx, n, 1, d); });
+            continue;
+        }
+        for (int y = 0; y < ny; y++)
+            read_units(nx, node_bytes, to + layer * z + row * y, stream,
+                       [&](int x, int n, double* d) { return eval(x, y, z, n, 1, 1, d); });
     }
 }
 
-void Readback::read(size_t units, size_t unit_bytes, void* out, hipStream_t stream,
-                    const std::function<hipError_t(size_t, size_t, double*)>& eval) {
+void Readback::read_units(size_t units, size_t unit_bytes, char* out, hipStream_t stream,
+                          const std::function<hipError_t(int, int, double*)>& eval) {
     const size_t total = units * unit_bytes;
-    if (total == 0) return;
-    std::lock_guard<std::mutex> one(m_);
-    if (total <= DIRECT) {
-        reserve(total, false);
-        hip_check(eval(0, units, (double*)pinned_), "field kernel");
-        hip_check(hipStreamSynchronize(stream), "read field");
-        std::memcpy(out, pinned_, total);
-        return;
-    }
     // four chunks, of 1 MB at least, so that small fields overlap too
     const size_t chunk = std::max(unit_bytes, std::min(CHUNK, std::max(CHUNK / 16, total / 4)));
     const size_t per = std::min(units, chunk / unit_bytes), chunks = (units + per - 1) / per;
-    reserve(per * unit_bytes, true);
-    for (hipEvent_t& e : done_)
-        if (!e) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event create");
+    // both buffers in one allocation, half as much again as before at least, so
+    // that a region that grows from read to read does not allocate on each
+    const size_t need = per * unit_bytes * std::min<size_t>(chunks, 2);
+    if (cap_ < need) {
+        const size_t want = std::max((need + 4095) / 4096 * 4096, cap_ + cap_ / 2);
+        cap_ = 0;
+        if (pinned_) (void)hipHostFree(pinned_);
+        pinned_ = nullptr;
+        hip_check(hipHostMalloc((void**)&pinned_, want, hipHostMallocDefault), "hipHostMalloc(field staging)");
+        cap_ = want;
+    }
     struct Drain {  // also a read that fails leaves nothing behind that writes to the buffers
         hipStream_t s;
         ~Drain() { (void)hipStreamSynchronize(s); }
-    } drain{stream};
+    };
+    if (chunks == 1) {
+        {
+            Drain drain{stream};
+            hip_check(eval(0, (int)units, (double*)pinned_), "field kernel");
+            hip_check(hipStreamSynchronize(stream), "read field");
+        }
+        std::memcpy(out, pinned_, total);
+        return;
+    }
+    for (hipEvent_t& e : done_)
+        if (!e) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventReleaseToSystem), "event create");
+    Drain drain{stream};
     // a thread for every 2 MB (for every 512 kB: U of 1024x256 400 us, not 311)
     Copier copier((unsigned)std::min<size_t>(8, 1 + total / (size_t(2) << 20)));
+    const auto buffer = [&](size_t c) { return pinned_ + (c & 1) * per * unit_bytes; };
     const auto start = [&](size_t c) {
-        const size_t b = c & 1, first = c * per, n = std::min(per, units - first);
-        hip_check(eval(first, n, (double*)(dev_ + b * dev_cap_)), "field kernel");
-        hip_check(hipMemcpyAsync(pinned_ + b * pinned_cap_, dev_ + b * dev_cap_, n * unit_bytes, hipMemcpyDeviceToHost, stream), "read field");
-        hip_check(hipEventRecord(done_[b], stream), "event record");
+        const size_t first = c * per, n = std::min(per, units - first);
+        hip_check(eval((int)first, (int)n, (double*)buffer(c)), "field kernel");
+        hip_check(hipEventRecord(done_[c & 1], stream), "event record");
     };
     start(0);
     for (size_t c = 0; c < chunks; c++) {
         if (c + 1 < chunks) start(c + 1);
-        const size_t b = c & 1, first = c * per, n = std::min(per, units - first);
-        hip_check(hipEventSynchronize(done_[b]), "read field");
-        copier.copy((char*)out + first * unit_bytes, pinned_ + b * pinned_cap_, n * unit_bytes);
+        const size_t first = c * per, n = std::min(per, units - first);
+        hip_check(hipEventSynchronize(done_[c & 1]), "read field");
+        copier.copy(out + first * unit_bytes, buffer(c), n * unit_bytes);
     }
 }
 

@@ -9,19 +9,22 @@
 
 namespace tclbx {
 
-// Two device buffers and two pinned host buffers of at most CHUNK bytes (or
-// one unit, where that is more), grown to what the reads so far needed and
-// freed with their owner.  A field is read in chunks: while one is evaluated
-// and copied to its pinned buffer, a few threads of this call copy the one
-// before into the caller's memory.  Reads of at most DIRECT bytes are
-// evaluated into the pinned buffer itself.  One read at a time; a second
-// thread's waits.
+// Two pinned host buffers of at most CHUNK bytes each, grown to what the reads
+// so far needed and freed with their owner; the field kernels write to them
+// over the host link.  A field is read in chunks: while one is evaluated into
+// its buffer, a few threads of this call copy the one before into the caller's
+// memory.  One read at a time; a second thread's waits.
 //
 // A large read is bound by the host link and by the first touch of the
 // caller's pages, which several threads share; a small one by calls.  Against
-// a device allocation per read and a copy to pageable memory (U of d3q19 256^3,
-// 403 MB, 38.0 -> 9.6 ms; of 256x128x128 9.7 -> 2.9; of 128x96x64, 19 MB,
-// 1.09 -> 0.67; of d2q9 1024x256, 6 MB, 403 -> 311 us; of 128x32 70 -> 22 us).
+// a device allocation per read and a copy to pageable memory, U of d3q19 256^3
+// (403 MB) 38.2 -> 8.7 ms, of 256x128x96 (75 MB) 7.5 -> 2.0, of 128x96x64 (19
+// MB) 1.38 -> 0.62, of 61x48x57 (4 MB) 0.29 -> 0.20.  The first read of a
+// lattice also pays for the pinned memory: 128x96x64 0.7 to 2.0 ms (1.4),
+// 61x48x57 0.25 to 0.3 (0.58), 32^3 85 us (64).  Through device buffers and
+// copies on the stream the steady reads took 10.5, 2.6, 0.67 and 0.25 ms, the
+// first of 128x96x64 1.6 to 3.2 and the first of a process, which sets up the
+// copies, 7 ms (now 2).
 class Readback {
 public:
     Readback() = default;
@@ -29,21 +32,22 @@ public:
     Readback(const Readback&) = delete;
     Readback& operator=(const Readback&) = delete;
 
-    static constexpr size_t CHUNK = size_t(16) << 20, DIRECT = size_t(128) << 10;
+    static constexpr size_t CHUNK = size_t(16) << 20;
 
-    // Reads `units` units (rows, layers) of `unit_bytes` bytes each into out:
-    // eval(first, count, dst) launches on `stream` what writes the units
-    // [first, first + count) to the device address dst.
-    void read(size_t units, size_t unit_bytes, void* out, hipStream_t stream,
-              const std::function<hipError_t(size_t, size_t, double*)>& eval);
+    // A box of nx x ny x nz nodes of node_bytes bytes each into out:
+    // eval(x, y, z, nx, ny, nz, dst) launches on `stream` what writes the part
+    // of the box from (x, y, z) on, of that size, to the device address dst.
+    using Eval = std::function<hipError_t(int, int, int, int, int, int, double*)>;
+    void read(int nx, int ny, int nz, size_t node_bytes, void* out, hipStream_t stream, const Eval& eval);
 
 private:
-    void reserve(size_t bytes, bool device);
+    // `units` units of unit_bytes (at most CHUNK) bytes each: eval(first, count, dst)
+    void read_units(size_t units, size_t unit_bytes, char* out, hipStream_t stream,
+                    const std::function<hipError_t(int, int, double*)>& eval);
     std::mutex m_;
-    char* dev_ = nullptr;     // two buffers of dev_cap_ bytes, one after the other
-    char* pinned_ = nullptr;  // two of pinned_cap_ bytes
+    char* pinned_ = nullptr;
     hipEvent_t done_[2] = {nullptr, nullptr};
-    size_t dev_cap_ = 0, pinned_cap_ = 0;
+    size_t cap_ = 0;
 };
 
 }  // namespace tclbx

@@ -1,6 +1,7 @@
 """Fields read in chunks: a whole field is what reads of its parts give, for
 sizes below the directly written ones, of one chunk, of many with a remainder
 and with a layer larger than a chunk."""
+import ctypes
 import threading
 
 import numpy as np
@@ -24,6 +25,7 @@ def parts(lat, q, rows):
     ("d3q19", "f64", 61, 48, 57),         # P: 1.3 MB, one chunk
     ("d3q27", "f32", 129, 97, 113),       # U: 34 MB by layers
     ("d3q19", "f16s", 1100, 1000, 3),     # a layer of U is 26 MB
+    ("d2q9_SRT", "f64", 800011, 6, 1),    # a row of U is 19 MB
 ])
 def test_whole_field_is_its_parts(model, storage, nx, ny, nz):
     say(f"reads {model} {storage} {nx}x{ny}x{nz}")
@@ -76,3 +78,31 @@ def test_batch_reads():
             lat.iterate(5)
             for q in ("U", lat.quantities[0]):
                 assert np.array_equal(batch.quantity(i, q), lat.quantity(q), equal_nan=True), q
+
+
+def free_device_memory():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert ctypes.CDLL("libamdhip64.so").hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_reads_keep_no_device_memory():
+    """A read leaves no device memory behind beyond what a few kB of launches
+    take, whatever the size of a layer: U of 1100x1000 is 26 MB a layer."""
+    say("device memory of reads")
+    tclb_amd.Lattice("d3q19", 8, 8, 8, "f16s").quantity("U")   # the runtime's own first needs
+    shape = (1100, 1000, 3)
+    batch = tclb_amd.Batch("d3q19", "f16s", capacity_bytes=1 << 29)
+    cid = batch.add_case(*shape)
+    lat = tclb_amd.Lattice("d3q19", *shape, "f16s")
+    flags = np.full(shape[::-1], lat.spec.flag("MRT"), np.uint16)
+    lat.set_flags(flags)
+    lat.init()
+    batch.set_flags(cid, flags)
+    batch.init_case(cid)
+    for x in (lat, batch):
+        x.iterate(2)
+    free = free_device_memory()
+    u, v = lat.quantity("U"), batch.quantity(cid, "U")
+    assert np.array_equal(u, v)
+    assert free - free_device_memory() <= 4 << 20
