@@ -43,21 +43,12 @@ template <class L> __host__ __device__ constexpr int ez_count(int ez) {
 template <class L> constexpr int march3d_slots = ez_count<L>(-1) + 2 * ez_count<L>(0) + 3 * ez_count<L>(1);
 
 // f stored: populations of a node rounded as the single step rounds its
-// stores, put(i, value) for each; with stochastic rounding direction 2j takes
-// word j of the node's stream and 2j + 1 word j << 16
+// stores, put(i, value) for each
 template <class S, class L, bool DEV, class PUT>
-__device__ __forceinline__ void store_node(const typename S::R* f, uint32_t w, PUT put) {
-    using R = typename S::R;
+__device__ __forceinline__ void store_node(const typename S::R* f, PUT put) {
+    static_assert(!S::stochastic, "the formats that march are not rounded stochastically");
 #pragma unroll
-    for (int i = 0; i < L::Q; i++) {
-        if constexpr (S::stochastic) {
-            const uint32_t r = (i & 1) ? w << 16 : w;
-            put(i, DEV ? S::unraw_sr(f[i], r) : S::put_sr(f[i], (R)L::w(i), r));
-            if (i & 1) w = xorshift32(w);
-        } else {
-            put(i, DEV ? S::unraw(f[i]) : S::put(f[i], (R)L::w(i)));
-        }
-    }
+    for (int i = 0; i < L::Q; i++) put(i, DEV ? S::unraw(f[i]) : S::put(f[i], (typename S::R)L::w(i)));
 }
 
 // Two plain steps of a column of tiles.  Block b owns a TX x TY tile of
@@ -154,12 +145,9 @@ __global__ void __launch_bounds__(TX * TY) k_march3d(StepArgs a, int tiles_x, in
             for (int i = 0; i < Q; i++) f[i] = DEV ? S::raw(u[i]) : S::get(u[i], (R)L::w(i));
             plain_node3d<MODEL, ST>(a, f, nt2);
             if (writes) {
-                uint32_t w = 0;
-                if constexpr (S::stochastic)
-                    w = sr_word0((unsigned)x + (unsigned)nx * (unsigned)y + layer * (unsigned)z2, sr_key(a.sr_step + 1u, a.sr_seed));
                 char* plane = (char*)a.fout + (size_t)z2 * layer * sizeof(T);
                 asm volatile("" : "+s"(plane));
-                store_node<S, L, DEV>(f, w, [&](int, T out) {
+                store_node<S, L, DEV>(f, [&](int, T out) {
                     *(gptr<T>)(plane + off[1][1]) = out;
                     plane += pbytes;
                     asm volatile("" : "+s"(plane));
@@ -168,11 +156,8 @@ __global__ void __launch_bounds__(TX * TY) k_march3d(StepArgs a, int tiles_x, in
         }
         if (it < layers + 2) {
             plain_node3d<MODEL, ST>(a, fn, nt0);
-            uint32_t w = 0;
-            if constexpr (S::stochastic)
-                w = sr_word0((unsigned)x + (unsigned)nx * (unsigned)y + layer * (unsigned)z, sr_key(a.sr_step, a.sr_seed));
             __syncthreads();
-            store_node<S, L, DEV>(fn, w, [&](int i, T out) {
+            store_node<S, L, DEV>(fn, [&](int i, T out) {
                 if (L::ez(i) < 0) own[ez_rank<L>(i) * NT] = out;
                 else if (L::ez(i) == 0) own[(NM + zc * NZ + ez_rank<L>(i)) * NT] = out;
                 else own[(NM + 2 * NZ + p0 * NP + ez_rank<L>(i)) * NT] = out;
