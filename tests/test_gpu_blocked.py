@@ -44,22 +44,27 @@ def test_marching_waves_are_bit_identical(model, storage, nx, ny, k):
         assert same(fa, b.get_f()), n
 
 
-@pytest.mark.parametrize("storage,sizes", [
-    ("f64", [(700, 601), (61, 500), (901, 800)]),   # marching waves
-    ("f64", [(75, 41), (20, 9), (130, 70)]),        # tiles, one case smaller than a tile
-    ("f16s", [(75, 41), (20, 9), (130, 70)]),
+@pytest.mark.parametrize("storage,sizes,sr", [
+    ("f64", [(700, 601), (61, 500), (901, 800)], False),      # marching waves, 4 steps
+    ("f64", [(2050, 1031), (61, 500), (1501, 1405)], False),  # 5 steps
+    ("f16s", [(2050, 1031), (61, 500), (1501, 1405)], True),  # 3, each keyed by its own iteration
+    ("f64", [(75, 41), (20, 9), (130, 70)], False),           # tiles, one case smaller than a tile
+    ("f16s", [(75, 41), (20, 9), (130, 70)], False),
 ])
-def test_blocked_batch_steps_are_bit_identical(storage, sizes):
+def test_blocked_batch_steps_are_bit_identical(storage, sizes, sr):
     """Every case of a batch steps as a lone lattice's single steps, through
     whole launches, rests, graph replays and a case that joins mid-run."""
-    say(f"blocked batch {storage} {sizes}")
+    say(f"blocked batch {storage} {sizes} sr={sr}")
     cases = [random_case("d2q9_drag", nx, ny, 1, seed=11 + i) for i, (nx, ny) in enumerate(sizes)]
     batch = tclb_amd.Batch("d2q9_drag", storage, 1 << 30)
     lats = []
     for c in cases:
         lat = c.build(storage)
         lat.temporal_blocking = 0
+        lat.set_block(256)   # the batch's: Globals are summed by block
         lats.append(lat)
+    for x in [batch] + lats if sr else []:
+        x.set_stochastic_rounding(True, seed=3)
     ids = [batch.add(c) for c in cases[:2]]
     batch.set_graph_steps(2)
     for step, n in enumerate((1, 7, 24)):
