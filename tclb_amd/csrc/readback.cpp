@@ -13,6 +13,8 @@
 namespace tclbx {
 
 namespace {
+constexpr size_t SMALL = size_t(128) << 10, HUGE_PAGE = size_t(2) << 20;
+
 // copies split over the calling thread and some of its own
 class Copier {
 public:
@@ -113,33 +115,31 @@ void Readback::read_units(size_t units, size_t unit_bytes, char* out, hipStream_
     // four chunks, of 1 MB at least, so that small fields overlap too
     const size_t chunk = std::max(unit_bytes, std::min(CHUNK, std::max(CHUNK / 16, total / 4)));
     const size_t per = std::min(units, chunk / unit_bytes), chunks = (units + per - 1) / per;
-    // both buffers in one allocation, half as much again as before at least, so
-    // that a region that grows from read to read does not allocate on each
-    const size_t need = per * unit_bytes * std::min<size_t>(chunks, 2);
+    // Both buffers in one allocation, whole huge pages unless small: in 4 kB
+    // pages the allocation and the first copy out of it cost about 0.5 ms each
+    // per 2 MB.  Sized by the chunk, not by the units that fit in it, so that a
+    // smaller field after a larger one fits.
+    const size_t need = chunks == 1 ? total : 2 * chunk, page = need > SMALL ? HUGE_PAGE : 4096;
     if (cap_ < need) {
-        const size_t want = std::max((need + 4095) / 4096 * 4096, cap_ + cap_ / 2);
+        const size_t want = (need + page - 1) / page * page;
         cap_ = 0;
         if (pinned_) (void)hipHostFree(pinned_);
         pinned_ = nullptr;
         hip_check(hipHostMalloc((void**)&pinned_, want, hipHostMallocDefault), "hipHostMalloc(field staging)");
         cap_ = want;
     }
-    struct Drain {  // also a read that fails leaves nothing behind that writes to the buffers
-        hipStream_t s;
-        ~Drain() { (void)hipStreamSynchronize(s); }
-    };
     if (chunks == 1) {
-        {
-            Drain drain{stream};
-            hip_check(eval(0, (int)units, (double*)pinned_), "field kernel");
-            hip_check(hipStreamSynchronize(stream), "read field");
-        }
+        hip_check(eval(0, (int)units, (double*)pinned_), "field kernel");
+        hip_check(hipStreamSynchronize(stream), "read field");
         std::memcpy(out, pinned_, total);
         return;
     }
     for (hipEvent_t& e : done_)
         if (!e) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventReleaseToSystem), "event create");
-    Drain drain{stream};
+    struct Drain {  // also a read that fails leaves nothing behind that writes to the buffers
+        hipStream_t s;
+        ~Drain() { (void)hipStreamSynchronize(s); }
+    } drain{stream};
     // a thread for every 2 MB (for every 512 kB: U of 1024x256 400 us, not 311)
     Copier copier((unsigned)std::min<size_t>(8, 1 + total / (size_t(2) << 20)));
     const auto buffer = [&](size_t c) { return pinned_ + (c & 1) * per * unit_bytes; };

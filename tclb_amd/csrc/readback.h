@@ -20,11 +20,11 @@ namespace tclbx {
 // a device allocation per read and a copy to pageable memory, U of d3q19 256^3
 // (403 MB) 38.2 -> 8.7 ms, of 256x128x96 (75 MB) 7.5 -> 2.0, of 128x96x64 (19
 // MB) 1.38 -> 0.62, of 61x48x57 (4 MB) 0.29 -> 0.20.  The first read of a
-// lattice also pays for the pinned memory: 128x96x64 0.7 to 2.0 ms (1.4),
-// 61x48x57 0.25 to 0.3 (0.58), 32^3 85 us (64).  Through device buffers and
-// copies on the stream the steady reads took 10.5, 2.6, 0.67 and 0.25 ms, the
-// first of 128x96x64 1.6 to 3.2 and the first of a process, which sets up the
-// copies, 7 ms (now 2).
+// lattice also pays for the pinned memory: 256^3 8.7 to 9.8 ms (38), 128x96x64
+// 1.0 to 1.2 (1.4 to 2.2), 61x48x57 0.26 to 0.75 (0.28 to 0.58, by the
+// runtime), 32^3 95 us (62).  Through device buffers and copies on the stream
+// the steady reads took 10.5, 2.6, 0.67 and 0.25 ms, and the first of a
+// process, which sets up the copies, up to 7 ms (now 1 to 2).
 class Readback {
 public:
     Readback() = default;
