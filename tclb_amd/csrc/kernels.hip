@@ -125,8 +125,9 @@ double weight(int model, int q) {
 // populations moved) are fitted to the times of 46 lattices, from 64x64 to
 // 4096x2048 and among them 4x262144, 57x20000 and 1000000x4, with single steps,
 // waves of k = 3 to 5 and tiles of k = 3 to 5 and 256 to 1024 nodes: within 6
-// to 15% (rms) of each, and the steps they choose take 2% longer than the best
-// of all on average (lines by size alone: 17%, up to 4.2 times).  us per step
+// to 15% (rms) of each, then moved a little so that the choices come closest to
+// the best of all: 1.2% behind on average (lines by size alone: 17%, up to 4.2
+// times).  us per step
 // of single steps, waves and tiles where sizes alone mislead: f32s 256x256 3.6,
 // 4.7 and, with k = 3 and 5, 2.5 and 1.8; 1500x1000 21.6, 8.1, 13.4; f16s
 // 4x262144, where a strip or tile wastes most of its columns, 10, 56, 18; f64
@@ -142,15 +143,15 @@ struct StepCost2d {
 static const StepCost2d& step_cost2d(int model, int storage, bool sr) {
     static const StepCost2d costs[2][4] = {
         // d2q9_SRT(_drag): f64, f32 and f32s, 16 bit, 16 bit with stochastic rounding
-        {{2.91, 0.181, 3.61, 0.127, 0, 0.85, 0.13, 0, 6.48, 0.0434, 0.0468, 0.317, 0.177},
-         {2.56, 0.186, 4.12, 0.227, 0, 0.0942, 0.035, 0.0932, 6.02, 0.0784, 0.0549, 0.196, 0.0326},
-         {2.64, 0.220, 3.70, 0.313, 0, 0.150, 0.070, 0.107, 6.94, 0.0424, 0.0471, 0.196, 0.0856},
-         {3.09, 0.218, 4.23, 0.242, 0, 0.170, 0.130, 0, 8.21, 0.0348, 0.0612, 0.226, 0.185}},
+        {{2.60, 0.183, 3.50, 0.117, 0, 1.09, 0.123, 0, 6.64, 0.0399, 0.0444, 0.303, 0.190},
+         {2.40, 0.157, 4.15, 0.191, 0, 0.0874, 0.0346, 0.124, 5.24, 0.0735, 0.0478, 0.195, 0.0254},
+         {3.32, 0.221, 4.35, 0.227, 0, 0.220, 0.0924, 0.0744, 5.92, 0.0342, 0.0410, 0.228, 0.0851},
+         {2.98, 0.267, 4.49, 0.306, 0, 0.192, 0.133, 0, 8.57, 0.0342, 0.0562, 0.241, 0.152}},
         // d2q9(_drag), the same
         {{3.09, 0.182, 1.91, 0.133, 0, 0.897, 0.156, 0.203, 7.54, 0.0261, 0.0499, 0.372, 0.244},
-         {2.79, 0.187, 3.65, 0.207, 0, 0.262, 0.0509, 0.128, 6.98, 0.0375, 0.0495, 0.282, 0.0891},
+         {2.83, 0.193, 3.41, 0.222, 0, 0.268, 0.0458, 0.128, 6.73, 0.0341, 0.0516, 0.268, 0.0793},
          {2.73, 0.192, 3.40, 0.284, 0, 0.217, 0.090, 0.116, 6.85, 0.0395, 0.0418, 0.196, 0.106},
-         {3.21, 0.191, 4.22, 0.222, 0, 0.196, 0.159, 0, 7.28, 0.0511, 0.020, 0.247, 0.220}}};
+         {3.04, 0.220, 4.34, 0.207, 0, 0.206, 0.184, 0, 6.76, 0.0608, 0.0222, 0.288, 0.241}}};
     const int f = storage == ST_F64 ? 0 : storage == ST_F32 || storage == ST_F32S ? 1 : sr ? 3 : 2;
     return costs[model == MODEL_D2Q9 || model == MODEL_D2Q9_DRAG][f];
 }
