@@ -317,7 +317,9 @@ def main():
             "nodes": N,
         },
         "roofline": {
-            "bound": "hbm",
+            # the march of two steps per launch has two waves per SIMD, which
+            # fill neither the vector units (49%) nor HBM (profiles/steps_per_launch.md)
+            "bound": "hbm" if r["steps_per_launch"] == 1 else "occupancy",
             "achieved": round(r["achieved_GBs"], 1),
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",

@@ -24,10 +24,10 @@ __device__ __forceinline__ typename S::T tb_stored(typename S::R v, int i, uint3
 }
 
 // Stores past the L2 (NT) where one round of blocks is the whole launch: the
-// launch then does not end with the L2's write-back (1024x128 in FP64, 4 steps
-// per launch: 3.39 us per step against 3.58); plain stores where there is more
+// launch then does not end with the L2's write-back (1024x128 in FP64, a launch
+// of 4 steps: 3.39 us per step against 3.58); plain stores where there is more
 // to overlap it with, whose partial lines at a tile's edge the L2 joins
-// (4096x2048, 4 steps: 128 us against 152).
+// (4096x2048 on tiles, 4 steps: 128 us against 152), and in batches.
 template <bool NT, class T> __device__ __forceinline__ void tb_store(T v, gptr<T> p) {
     if constexpr (NT) __builtin_nontemporal_store(v, p);
     else *p = v;
