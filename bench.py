@@ -318,7 +318,7 @@ def main():
         },
         "roofline": {
             # the march of two steps per launch has two waves per SIMD, which
-            # fill neither the vector units (49%) nor HBM (profiles/steps_per_launch.md)
+            # fill neither the vector units (49%) nor HBM; counters under profiles/
             "bound": "hbm" if r["steps_per_launch"] == 1 else "occupancy",
             "achieved": round(r["achieved_GBs"], 1),
             "peak": HBM_PEAK_GBS,

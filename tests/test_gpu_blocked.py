@@ -19,13 +19,14 @@ def same(a, b):
 @pytest.mark.parametrize("model,storage,nx,ny,k", [
     ("d2q9_SRT", "f64", 1031, 1021, 2),         # 1,031 = 16 strips of 62 and 39 columns
     ("d2q9_drag", "f64", 1031, 1021, 4),
-    ("d2q9_SRT_drag", "f64", 57, 18500, 5),
+    ("d2q9_SRT_drag", "f64", 57, 18500, 5),     # a second strip of one column: tiles take it
     ("d2q9_SRT_drag", "f64", 50, 21000, 5),     # narrower than a strip of 56: its halo wraps onto itself
-    ("d2q9", "f16s", 2053, 2049, 3),
+    ("d2q9", "f16s", 2053, 2049, 3),            # tiles, with stochastic rounding's cost
+    ("d2q9_SRT", "f16s", 2053, 2049, 3),
     ("d2q9_SRT", "f32s", 70001, 61, 5),         # rows that a segment of 12 does not divide
 ])
 def test_marching_waves_are_bit_identical(model, storage, nx, ny, k):
-    """Lattices past the line where k <= 5 steps per launch march, against
+    """Lattices whose k <= 5 steps per launch march (two take tiles), against
     single steps: a whole launch, a shorter rest of steps, stochastic
     rounding in the 16-bit format."""
     say(f"marching waves {model} {storage} {nx}x{ny} k={k}")
